@@ -180,22 +180,28 @@ def get_block_map(q: torch.Tensor, k: torch.Tensor, topk_ratio: float, BLKQ: int
 
 
 def sparse_attention(q, k, v, topk_ratio: float, blk: int = 64, force_diag: bool = False,
-                     smooth_k: bool = True, pooled=None):
+                     smooth_k: bool = True, pooled=None, seq_major: bool = False):
     """[1,H,S,D] -> [1,H,S,D] block-sparse attention (SLA sparse branch only; h3_sla:226-235).
 
     Native block sizes run on the block LUT; the others on the tile LUT
     built from the block map.  `pooled`: block means from the prologue (see
-    get_block_map).
+    get_block_map).  `seq_major`: the kernel writes O as [1,S,H,D] memory and
+    the result is its [1,H,S,D] view, so that a caller who wants [1,S,H*D]
+    (the layer's output projection) reshapes it without a copy.
     """
     blk = check_block(blk)
     out_dtype = q.dtype
     q16, k16, v16 = (t.to(torch.bfloat16) for t in (q, k, v))
     native = blk in ops.NATIVE_BLOCKS
+    out = None
+    if seq_major:
+        B, H, S, D = q16.shape
+        out = torch.empty((B, S, H, D), dtype=torch.bfloat16, device=q16.device).transpose(1, 2)
     bmap, lut, counts = get_block_map(q16, k16, topk_ratio, blk, blk, force_diag=force_diag,
                                       smooth_k=smooth_k, want_map=not native, pooled=pooled)
     if native:
-        o = ops.attn_fwd_blocksparse(q16, k16, v16, lut, counts, blk, blk)
+        o = ops.attn_fwd_blocksparse(q16, k16, v16, lut, counts, blk, blk, out=out)
     else:
         tlut, tcnt = ops.block_map_to_tile_lut(bmap, blk, blk, q16.shape[2], k16.shape[2])
-        o = ops.attn_fwd_blocksparse_tiles(q16, k16, v16, tlut, tcnt)
+        o = ops.attn_fwd_blocksparse_tiles(q16, k16, v16, tlut, tcnt, out=out)
     return o.to(out_dtype)
