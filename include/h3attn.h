@@ -254,6 +254,14 @@ int h3a_block_map_to_lut(const uint8_t *block_map, int B, int H, int nq, int nk,
                          h3a_stream_t stream);
 
 /*
+ * The LUT width a block map needs: partial[i], i < partials, are maxima of the
+ * map's row sums (bytes added as they are) over disjoint sets of rows; their
+ * maximum is the largest row sum, the max_k_blocks that keeps every block.
+ */
+int h3a_block_map_row_max(const uint8_t *block_map, int B, int H, int nq, int nk, int32_t *partial,
+                          int partials, h3a_stream_t stream);
+
+/*
  * Block means for the block map: out[b,h,j,:] = mean of x[b,h,r,:] over the
  * valid rows r of block j (blocks of blk rows; the last may be partial).
  * x: bf16 [B,H,S,D] with strides {batch, head, seq} (elements), D == 128.

@@ -447,6 +447,17 @@ int h3a_block_map_to_lut(const uint8_t *block_map, int B, int H, int nq, int nk,
   return launch_block_map_to_lut(block_map, B, H, nq, nk, lut, counts, max_k_blocks, as_stream(stream));
 }
 
+int h3a_block_map_row_max(const uint8_t *block_map, int B, int H, int nq, int nk, int32_t *partial, int partials,
+                          h3a_stream_t stream) {
+  clear_error();
+  if (!block_map || !partial) return fail(H3A_ERR_INVALID_ARG, "null pointer");
+  if (B <= 0 || H <= 0 || nq <= 0 || nk <= 0)
+    return fail(H3A_ERR_INVALID_ARG, "sizes must be positive (B=%d H=%d nq=%d nk=%d)", B, H, nq, nk);
+  if (partials <= 0 || partials > (1 << 20))
+    return fail(H3A_ERR_INVALID_ARG, "partials %d outside [1, %d]", partials, 1 << 20);
+  return launch_block_map_row_max(block_map, B, H, nq, nk, partial, partials, as_stream(stream));
+}
+
 int h3a_block_pool(const void *x, int B, int H, int S, int D, const int64_t strides[3], int blk,
                    float *out, h3a_stream_t stream) {
   clear_error();

@@ -1462,24 +1462,72 @@ __global__ void __launch_bounds__(64) test_pv_kernel(const uint16_t *P, const ui
 }
 
 // ---------------------------------------------------------------------------
-// Block map [B,H,nq,nk] (0/1 bytes) -> ascending LUT + counts, one thread per row.
+// Block map [B,H,nq,nk] (0/1 bytes) -> ascending LUT + counts, one wave per row:
+// lane l reads block 64c + l (64 contiguous bytes per wave access) and a ballot
+// gives every kept block its place.  Latency-bound (a load, a ballot and a store
+// per 64 blocks), so four chunks' loads are in flight at a time; with one thread
+// per row the walk was a chain of nk byte loads 64 rows apart.  3584 rows of 64
+// blocks: 3.4 us against 19.6.
+constexpr int kMapUnroll = 4;
 __global__ void __launch_bounds__(256) block_map_to_lut_kernel(const uint8_t *map, int64_t rows,
                                                                int nk, int32_t *lut,
                                                                int32_t *counts, int max_k) {
-  const int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (row >= rows) return;
-  const uint8_t *m = map + row * nk;
-  int32_t *out = lut + row * max_k;
-  int c = 0;
-  for (int j = 0; j < nk; ++j) {
-    if (m[j] != 0) {
-      if (c < max_k) out[c] = j;
-      ++c;
+  const int lane = threadIdx.x & 63;
+  const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));  // lanes < this one
+  for (int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); row < rows; row += (int64_t)gridDim.x * 4) {
+    const uint8_t *m = map + row * nk;
+    int32_t *out = lut + row * max_k;
+    int c = 0;
+    for (int j0 = 0; j0 < nk; j0 += 64 * kMapUnroll) {
+      uint8_t v[kMapUnroll];
+#pragma unroll
+      for (int u = 0; u < kMapUnroll; ++u) {
+        const int j = j0 + 64 * u + lane;
+        v[u] = j < nk ? m[j] : (uint8_t)0;
+      }
+#pragma unroll
+      for (int u = 0; u < kMapUnroll; ++u) {
+        const uint64_t kept = __builtin_amdgcn_ballot_w64(v[u] != 0);
+        const int pos = c + __builtin_popcountll(kept & below);
+        if (v[u] != 0 && pos < max_k) out[pos] = j0 + 64 * u + lane;
+        c += __builtin_popcountll(kept);
+      }
     }
+    const int kept = c < max_k ? c : max_k;
+    for (int j = kept + lane; j < max_k; j += 64) out[j] = -1;
+    if (lane == 0) counts[row] = kept;
   }
-  const int kept = c < max_k ? c : max_k;
-  for (int j = kept; j < max_k; ++j) out[j] = -1;
-  counts[row] = kept;
+}
+
+// The largest row sum of a block map (the LUT width its rows need), as one
+// partial maximum per workgroup: a workgroup takes rows 4*blockIdx.x + wave,
+// stepping by the grid.
+__global__ void __launch_bounds__(256) block_map_row_max_kernel(const uint8_t *map, int64_t rows, int nk,
+                                                                int32_t *partial) {
+  __shared__ int32_t wave_max[4];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int best = 0;
+  for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < rows; row += (int64_t)gridDim.x * 4) {
+    const uint8_t *m = map + row * nk;
+    int n = 0;
+    for (int j0 = 0; j0 < nk; j0 += 64 * kMapUnroll) {
+#pragma unroll
+      for (int u = 0; u < kMapUnroll; ++u) {
+        const int j = j0 + 64 * u + lane;
+        n += j < nk ? (int)m[j] : 0;
+      }
+    }
+#pragma unroll
+    for (int s = 32; s >= 1; s >>= 1) n += __shfl_xor(n, s);
+    best = n > best ? n : best;
+  }
+  if (lane == 0) wave_max[wave] = best;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 1; w < 4; ++w) best = wave_max[w] > best ? wave_max[w] : best;
+    partial[blockIdx.x] = best;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1753,10 +1801,17 @@ int launch_attn_sparse(const AttnArgs &a, int blk_q, hipStream_t s, bool tiles) 
 int launch_block_map_to_lut(const uint8_t *map, int B, int H, int nq, int nk, int32_t *lut,
                             int32_t *counts, int max_k_blocks, hipStream_t s) {
   const int64_t rows = (int64_t)B * H * nq;
-  const int64_t blocks = (rows + 255) / 256;
-  hipLaunchKernelGGL(block_map_to_lut_kernel, dim3((unsigned)blocks), dim3(256), 0, s, map, rows, nk,
-                     lut, counts, max_k_blocks);
+  const int64_t blocks = (rows + 3) / 4 < (1 << 20) ? (rows + 3) / 4 : (1 << 20);
+  hipLaunchKernelGGL(block_map_to_lut_kernel, dim3((unsigned)blocks), dim3(256), 0, s, map, rows, nk, lut, counts,
+                     max_k_blocks);
   return check_launch("block_map_to_lut_kernel");
+}
+
+int launch_block_map_row_max(const uint8_t *map, int B, int H, int nq, int nk, int32_t *partial, int partials,
+                             hipStream_t s) {
+  hipLaunchKernelGGL(block_map_row_max_kernel, dim3((unsigned)partials), dim3(256), 0, s, map, (int64_t)B * H * nq,
+                     nk, partial);
+  return check_launch("block_map_row_max_kernel");
 }
 
 int launch_test_qk(const uint16_t *Q, const uint16_t *K, float *S, hipStream_t s) {

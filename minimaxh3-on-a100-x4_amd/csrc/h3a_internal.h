@@ -96,6 +96,8 @@ int launch_attn_sparse_split(const AttnArgs &a, int blk_q, const SplitPlan &plan
                              bool tiles = false);
 int launch_block_map_to_lut(const uint8_t *map, int B, int H, int nq, int nk, int32_t *lut,
                             int32_t *counts, int max_k_blocks, hipStream_t s);
+int launch_block_map_row_max(const uint8_t *map, int B, int H, int nq, int nk, int32_t *partial, int partials,
+                             hipStream_t s);
 int launch_block_map_to_tile_lut(const uint8_t *map, int B, int H, int Sq, int Skv, int blk_q, int blk_k,
                                  int32_t *lut, int32_t *counts, int max_tiles, hipStream_t s);
 int launch_lut_to_block_map(const int32_t *lut, const int32_t *counts, int B, int H, int nq, int nk,
