@@ -62,4 +62,17 @@ __host__ __device__ __forceinline__ int lut_stage_key0_magic(int t, int kb, int 
   return (int)(key0 < (uint32_t)Skv ? key0 : (uint32_t)Skv);
 }
 
+// Key block of 16-key unit u (u < 2^18: the units a tile LUT can name) at
+// blk_k = 16 b keys: u / b = (u * magic) >> 36 with magic = ceil(2^36 / b).
+// Exact for b <= 2^18: the product exceeds 2^36 u / b by u * (magic * b - 2^36) / b
+// < 2^36 / b, too little to reach the next integer.  Larger b (every u in block
+// 0) take the magic of 2^18.
+__host__ __device__ __forceinline__ uint64_t unit_magic(int blk_k) {
+  const uint64_t b = (uint64_t)(blk_k / 16) < (1u << 18) ? (uint64_t)(blk_k / 16) : (1u << 18);
+  return (((uint64_t)1 << 36) + b - 1) / b;
+}
+__host__ __device__ __forceinline__ int block_of_unit(int u, uint64_t magic) {
+  return (int)(((uint64_t)(uint32_t)u * magic) >> 36);
+}
+
 }  // namespace h3a

@@ -4,7 +4,7 @@ import pytest
 import torch
 
 import h3attn
-from h3attn import sla
+from h3attn import ops, sla
 
 pytestmark = pytest.mark.gpu
 
@@ -36,3 +36,28 @@ def test_block_map_to_lut_chunk_edges(gpu, rows, nk, fill):
             nz = m[0, 0, r].nonzero().flatten()[:k].int()
             want[0, 0, r, :len(nz)] = nz
         assert torch.equal(lut.cpu(), want) and torch.equal(cnt.cpu(), counts.clamp(max=k))
+
+
+@pytest.mark.parametrize("blk_q,blk_k,Sq,Skv", [(16, 16, 130, 4113), (48, 80, 1000, 2065), (96, 96, 65, 8200),
+                                                (256, 240, 700, 2048), (112, 32, 500, 31), (1040, 1 << 21, 3000, 777)])
+def test_tile_lut_chunk_and_slice_edges(gpu, blk_q, blk_k, Sq, Skv):
+    """Tile LUTs against their element mask: shared map rows, split columns, ragged ends, several
+    256-column chunks."""
+    torch.manual_seed(Sq)
+    nq, nk = -(-Sq // blk_q), -(-Skv // blk_k)
+    m = (torch.rand(1, 2, nq, nk) < 0.4).to(torch.uint8)
+    lut, cnt = ops.block_map_to_tile_lut(m.to(gpu), blk_q, blk_k, Sq, Skv)
+    nsub, ncols = -(-Sq // 64), -(-Skv // 32)
+    rows, keys = torch.arange(4 * nsub) * 16, torch.arange(2 * ncols) * 16
+    sub = m[:, :, (rows // blk_q).clamp(max=nq - 1)][..., (keys // blk_k).clamp(max=nk - 1)].bool()
+    sub &= (rows < Sq)[:, None] & (keys < Skv)
+    bit = torch.tensor([[1 << (2 * i + j) for j in range(2)] for i in range(4)])
+    mask = (sub.view(1, 2, nsub, 4, ncols, 2) * bit[:, None, :]).sum((3, 5))
+    lut, cnt = lut.cpu(), cnt.cpu()
+    assert torch.equal(cnt.long(), (mask != 0).sum(-1))
+    for h in range(2):
+        for qs in range(nsub):
+            cols = mask[0, h, qs].nonzero().flatten()
+            want = torch.full((ncols,), -1, dtype=torch.int32)
+            want[:len(cols)] = ((cols << 8) | mask[0, h, qs, cols]).int()
+            assert torch.equal(lut[0, h, qs], want)
