@@ -13,8 +13,9 @@
 // (1 KB contiguous in the fused QKV layout).  The token's RoPE matrices and
 // the two weight vectors are loaded into registers once per wave and reused
 // for all 2 x HPW rows; the chunk's row loads are issued before any math.  The sum of squares
-// is reduced across the 16 lanes with xor shuffles; the RoPE partner dims
-// (i, i+rot/2) sit rot/16 lanes apart and are fetched with one shuffle each.
+// is reduced across the 16 lanes with DPP moves; the RoPE partner dims
+// (i, i+rot/2) sit rot/16 lanes apart: a DPP rotation at rot = 128, else one
+// shuffle each.
 #include "h3a_device.h"
 #include "h3a_internal.h"
 
@@ -22,11 +23,25 @@ namespace h3a {
 
 constexpr int kRopeD = 128;
 
+// v of another lane of the same 16-lane row, in the VALU (no LDS round trip as
+// a shuffle takes).
+template <int CTRL>
+__device__ __forceinline__ float dpp_row(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+constexpr int kDppXor1 = 0xB1;         // quad_perm [1,0,3,2]
+constexpr int kDppXor2 = 0x4E;         // quad_perm [2,3,0,1]
+constexpr int kDppHalfMirror = 0x141;  // lane i of 8 <- 7 - i
+constexpr int kDppMirror = 0x140;      // lane i of 16 <- 15 - i
+constexpr int kDppRor8 = 0x128;        // lane i of 16 <- i ^ 8
+
+// Sum over the 16 lanes of a row, on all of them.  Once the lanes of a quad (of
+// 8) hold the same sum, a mirror pairs them as an xor with 4 (8) would.
 __device__ __forceinline__ float group16_sum(float v) {
-  v += __shfl_xor(v, 1, 16);
-  v += __shfl_xor(v, 2, 16);
-  v += __shfl_xor(v, 4, 16);
-  v += __shfl_xor(v, 8, 16);
+  v += dpp_row<kDppXor1>(v);
+  v += dpp_row<kDppXor2>(v);
+  v += dpp_row<kDppHalfMirror>(v);
+  v += dpp_row<kDppMirror>(v);
   return v;
 }
 
@@ -51,9 +66,23 @@ __device__ __forceinline__ u32x4 pack8(const float (&x)[8]) {
 // non-temporal stores changed nothing.
 __host__ __device__ constexpr int rope_heads_per_wave(int H) { return H % 28 == 0 ? 28 : 16; }
 
-// y = rmsnorm(x) * w, then rotate pairs (i, i+rot/2) with the lane's 2x2 matrices.
+// The lane's half of its token's 2x2 matrices: lanes of the first rotated half
+// (c < nh) apply the first row (R00, R01), their partners the second (R10, R11).
+// Lanes past the rotated dims hold nothing.
+__device__ __forceinline__ void load_rope(float2 (&R)[8], const float *rope_row, int c, int nh) {
+  if (c < 2 * nh) {
+    const float *p = rope_row + (c < nh ? c * 32 : (c - nh) * 32 + 2);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) R[e] = *(const float2 *)(p + 4 * e);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) R[e] = float2{0.f, 1.f};
+  }
+}
+
+// y = rmsnorm(x) * w, then rotate pairs (i, i+rot/2) with the lane's matrix rows.
 __device__ __forceinline__ void norm_rope_row(float (&x)[8], const float (&w)[8], float eps,
-                                              const float4 (&R)[8], int c, int rot) {
+                                              const float2 (&R)[8], int c, int nh) {
   float ss = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) ss = fmaf(x[e], x[e], ss);
@@ -62,17 +91,20 @@ __device__ __forceinline__ void norm_rope_row(float (&x)[8], const float (&w)[8]
 #pragma unroll
   for (int e = 0; e < 8; ++e) x[e] = x[e] * r * w[e];
 
-  const int nh = rot >> 4;  // lanes holding the first half of the rotated dims
   const bool first = c < nh;
   const bool rotated = c < 2 * nh;
-  const int partner = first ? c + nh : (rotated ? c - nh : c);
   float xp[8];
+  if (nh == 8) {  // rot = 128: the partner is 8 lanes away
 #pragma unroll
-  for (int e = 0; e < 8; ++e) xp[e] = __shfl(x[e], partner, 16);
+    for (int e = 0; e < 8; ++e) xp[e] = dpp_row<kDppRor8>(x[e]);
+  } else {
+    const int partner = first ? c + nh : (rotated ? c - nh : c);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) xp[e] = __shfl(x[e], partner, 16);
+  }
   if (rotated) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      x[e] = first ? fmaf(R[e].x, x[e], R[e].y * xp[e]) : fmaf(R[e].z, xp[e], R[e].w * x[e]);
+    for (int e = 0; e < 8; ++e) x[e] = fmaf(R[e].x, first ? x[e] : xp[e], R[e].y * (first ? xp[e] : x[e]));
   }
 }
 
@@ -91,16 +123,9 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_kernel(RopeArgs a) {
   float wq[8], wk[8];
   unpack8(*(const u32x4 *)(a.qw + c * 8), wq);
   unpack8(*(const u32x4 *)(a.kw + c * 8), wk);
-  float4 R[8];
+  float2 R[8];
   const int nh = a.rot >> 4;
-  if (c < 2 * nh) {
-    const float *rope_row = a.rope + b * a.rsb + s * a.rss + (c < nh ? c : c - nh) * 8 * 4;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) R[e] = *(const float4 *)(rope_row + e * 4);
-  } else {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) R[e] = float4{1.f, 0.f, 0.f, 1.f};
-  }
+  load_rope(R, a.rope + b * a.rsb + s * a.rss, c, nh);
 
   uint16_t *qrow = a.q + b * a.qsb + s * a.qss + c * 8;
   uint16_t *krow = a.k + b * a.ksb + s * a.kss + c * 8;
@@ -119,8 +144,8 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_kernel(RopeArgs a) {
     float xq[8], xk[8];
     unpack8(qv[i], xq);
     unpack8(kv[i], xk);
-    norm_rope_row(xq, wq, a.eps, R, c, a.rot);
-    norm_rope_row(xk, wk, a.eps, R, c, a.rot);
+    norm_rope_row(xq, wq, a.eps, R, c, nh);
+    norm_rope_row(xk, wk, a.eps, R, c, nh);
     if (heads[i] < a.H) {
       *(u32x4 *)(qrow + heads[i] * a.qsh) = pack8(xq);
       *(u32x4 *)(krow + heads[i] * a.ksh) = pack8(xk);
@@ -137,8 +162,14 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_kernel(RopeArgs a) {
 // scaled by 1/rows: block_pool_kernel's lane rg sums rows rg, rg+4, ... in
 // order and combines the four lane groups in that association, so the means
 // are equal to its output bit for bit, and the selection made from them is
-// the same.
-template <int kHeadsPerWave>
+// the same.  Bound by HBM at full size and by the latency of a wave's serial
+// tokens at small ones, so the loads of the next kDepth tokens are in flight
+// while one is computed (they come before its stores, which the compiler cannot
+// reorder) and the cross-lane steps stay in the VALU.  Per call, against loads,
+// LDS shuffles and stores token by token: H=14 S=4104 45.1 -> 27.8 us, H=56 S=4104
+// 67.2 -> 55.8, H=28 S=42120 (blocks of 96) 299 -> 269, H=56 S=42120 510 -> 502
+// (4.9 TB/s; a 2 GiB copy moves 5.0 on the same card).
+template <int kHeadsPerWave, int kDepth>
 __global__ void __launch_bounds__(256) qk_rmsnorm_rope_pool_kernel(RopeArgs a, int blk, int nb, float *pq,
                                                                    float *pk) {
   static_assert(kHeadsPerWave % 4 == 0, "four 16-lane groups per wave");
@@ -146,7 +177,8 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_pool_kernel(RopeArgs a, i
   // Partial sums of waves 1 and 3 (slots 0 and 1), then of wave 2 (slot 0):
   // [slot][step][q,k][lane] of 8 floats.
   __shared__ __attribute__((aligned(16))) float xch[2][kSteps][2][64][8];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, grp = lane >> 4, c = lane & 15;
+  const int tid = threadIdx.x, lane = tid & 63, grp = lane >> 4, c = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nchunk = (a.H + kHeadsPerWave - 1) / kHeadsPerWave;
   const int chunk = (int)(blockIdx.x % nchunk);
   const int64_t bj = blockIdx.x / nchunk;
@@ -167,33 +199,39 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_pool_kernel(RopeArgs a, i
 #pragma unroll
     for (int e = 0; e < 8; ++e) sq[i][e] = sk[i][e] = 0.f;
 
-  for (int t = wave; t < rows; t += 4) {
-    const int s = r0 + t;
-    float4 R[8];
-    if (c < 2 * nh) {
-      const float *rope_row = a.rope + b * a.rsb + s * a.rss + (c < nh ? c : c - nh) * 8 * 4;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) R[e] = *(const float4 *)(rope_row + e * 4);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) R[e] = float4{1.f, 0.f, 0.f, 1.f};
-    }
-    uint16_t *qrow = a.q + b * a.qsb + s * a.qss + c * 8;
-    uint16_t *krow = a.k + b * a.ksb + s * a.kss + c * 8;
-    u32x4 qv[kSteps], kv[kSteps];
+  // This wave's tokens wave, wave + 4, ...: a ring of kDepth tokens' loads in
+  // flight, each slot refilled once its token is done.  Loads past the wave's
+  // last token repeat it (its own rows), so they need no branch.
+  const int mine = (rows - wave + 3) / 4;
+  struct Token {
+    float2 R[8];
+    u32x4 q[kSteps], k[kSteps];
+  };
+  Token ring[kDepth];
+  auto token_of = [&](int n) __attribute__((always_inline)) { return r0 + wave + 4 * (n < mine ? n : mine - 1); };
+  auto load = [&](Token &in, int n) __attribute__((always_inline)) {
+    const int s = token_of(n);
+    load_rope(in.R, a.rope + b * a.rsb + s * a.rss, c, nh);
+    const uint16_t *qrow = a.q + b * a.qsb + s * a.qss + c * 8;
+    const uint16_t *krow = a.k + b * a.ksb + s * a.kss + c * 8;
 #pragma unroll
     for (int i = 0; i < kSteps; ++i) {
       const int hc = heads[i] < a.H ? heads[i] : a.H - 1;  // past-the-end groups store nothing
-      qv[i] = *(const u32x4 *)(qrow + hc * a.qsh);
-      kv[i] = *(const u32x4 *)(krow + hc * a.ksh);
+      in.q[i] = *(const u32x4 *)(qrow + hc * a.qsh);
+      in.k[i] = *(const u32x4 *)(krow + hc * a.ksh);
     }
+  };
+  auto process = [&](const Token &in, int n) __attribute__((always_inline)) {
+    const int s = token_of(n);
+    uint16_t *qrow = a.q + b * a.qsb + s * a.qss + c * 8;
+    uint16_t *krow = a.k + b * a.ksb + s * a.kss + c * 8;
 #pragma unroll
     for (int i = 0; i < kSteps; ++i) {
       float xq[8], xk[8];
-      unpack8(qv[i], xq);
-      unpack8(kv[i], xk);
-      norm_rope_row(xq, wq, a.eps, R, c, a.rot);
-      norm_rope_row(xk, wk, a.eps, R, c, a.rot);
+      unpack8(in.q[i], xq);
+      unpack8(in.k[i], xk);
+      norm_rope_row(xq, wq, a.eps, in.R, c, nh);
+      norm_rope_row(xk, wk, a.eps, in.R, c, nh);
       const u32x4 oq = pack8(xq), ok = pack8(xk);
       if (heads[i] < a.H) {
         *(u32x4 *)(qrow + heads[i] * a.qsh) = oq;
@@ -206,6 +244,17 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_pool_kernel(RopeArgs a, i
       for (int e = 0; e < 8; ++e) {
         sq[i][e] += yq[e];
         sk[i][e] += yk[e];
+      }
+    }
+  };
+  if (mine > 0) {
+#pragma unroll
+    for (int d = 0; d < kDepth; ++d) load(ring[d], d);
+    for (int n = 0; n < mine; n += kDepth) {
+#pragma unroll
+      for (int d = 0; d < kDepth; ++d) {
+        if (n + d < mine) process(ring[d], n + d);
+        load(ring[d], n + d + kDepth);
       }
     }
   }
@@ -248,11 +297,23 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_pool_kernel(RopeArgs a, i
   }
 }
 
+// Heads per workgroup.  A workgroup's waves walk their share of the block's
+// tokens one after another, so with fewer 8-head workgroups than CUs the launch
+// takes as long as one walk: 4-head chunks double the workgroups and shorten each
+// step.  Measured with 8 / 4 heads: 28.6 / 21.0 us at H=4 S=1024 (16 workgroups of
+// 8 heads), 33.3 / 27.8 at H=14 S=4104 (130), but 55.8 / 79.0 at H=56 S=4104 (455)
+// and 490 / 655 at H=56 S=42120 (4613), where 2 KiB per access of a token's q or k
+// against 1 KiB decides.
+constexpr int64_t kPoolWideWgs = 256;
 int launch_qk_rmsnorm_rope_pool(const RopeArgs &a, int blk, float *pq, float *pk, hipStream_t s) {
-  constexpr int kHpw = 8;
   const int nb = (a.S + blk - 1) / blk;
-  const int64_t wgs = (int64_t)a.B * nb * ((a.H + kHpw - 1) / kHpw);
-  hipLaunchKernelGGL(qk_rmsnorm_rope_pool_kernel<kHpw>, dim3((unsigned)wgs), dim3(256), 0, s, a, blk, nb, pq, pk);
+  const int64_t blocks = (int64_t)a.B * nb;
+  if (blocks * ((a.H + 7) / 8) < kPoolWideWgs)
+    hipLaunchKernelGGL((qk_rmsnorm_rope_pool_kernel<4, 2>), dim3((unsigned)(blocks * ((a.H + 3) / 4))), dim3(256),
+                       0, s, a, blk, nb, pq, pk);
+  else
+    hipLaunchKernelGGL((qk_rmsnorm_rope_pool_kernel<8, 1>), dim3((unsigned)(blocks * ((a.H + 7) / 8))), dim3(256),
+                       0, s, a, blk, nb, pq, pk);
   return check_launch("qk_rmsnorm_rope_pool_kernel");
 }
 

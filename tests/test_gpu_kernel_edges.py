@@ -61,3 +61,25 @@ def test_tile_lut_chunk_and_slice_edges(gpu, blk_q, blk_k, Sq, Skv):
             want = torch.full((ncols,), -1, dtype=torch.int32)
             want[:len(cols)] = ((cols << 8) | mask[0, h, qs, cols]).int()
             assert torch.equal(lut[0, h, qs], want)
+
+
+@pytest.mark.parametrize("S,H,blk,rot", [(63, 3, 64, 128), (64, 4, 64, 64), (65, 8, 64, 128), (1, 1, 64, 128),
+                                         (130, 14, 48, 96), (4104, 56, 64, 128), (2100, 60, 16, 32)])
+def test_pooled_prologue_tokens_heads_edges(gpu, S, H, blk, rot):
+    """The pooling prologue in 4-head and 8-head workgroups, ragged heads and last blocks of fewer tokens
+    than waves: its rows and means equal the plain prologue's and block_pool's bit for bit."""
+    torch.manual_seed(S)
+    qkv = torch.randn(S, 3 * H * 128, device=gpu).bfloat16()
+    rope = torch.randn(1, S, 1, rot // 2, 2, 2, device=gpu)
+    w = [torch.randn(128, device=gpu).bfloat16() for _ in range(2)]
+    got, want = qkv.clone(), qkv.clone()
+
+    def heads(x):
+        f = x.view(1, S, 3, H, 128)
+        return f[:, :, 0], f[:, :, 1]
+
+    means = ops.qk_rmsnorm_rope_(*heads(got), rope, *w, pool_blk=blk)
+    ops.qk_rmsnorm_rope_(*heads(want), rope, *w)
+    assert torch.equal(got, want)
+    for m, x in zip(means, heads(want)):
+        assert torch.equal(m, ops.block_pool(x.transpose(1, 2), blk))
