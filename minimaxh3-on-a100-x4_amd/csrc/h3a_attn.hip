@@ -8,7 +8,7 @@
 // :405-420), O = acc / l with row-guarded stores (:443-457).  How it is
 // computed is CDNA4-specific:
 //
-//  * Each wave keeps 32 query rows as the B operand of
+//  * Each wave keeps 32 query rows (fetched through LDS, QTile) as the B operand of
 //    v_mfma_f32_32x32x16_bf16 in VGPRs and produces the score tile
 //    transposed, S^T = K Q^T, so every lane owns a single query row (column
 //    l%32) and 32 of the 64 keys of a stage.  That layout is already the B
@@ -694,6 +694,42 @@ struct PingPongLds {
   static constexpr int NG = kSparse ? 2 : 1;  // K/V streams: one per group (sparse)
   uint16_t k[NG][2][kKE];
   uint16_t v[NG][2][kVE];
+  uint16_t q[kSparse ? 8 : 256 * kD];  // dense: the query tile (see QTile)
+};
+
+// A wave's 32 query rows on their way to registers: fetched by LDS DMA in whole
+// rows (instruction i: rows 4i .. 4i+3) into a 32-row tile in the K layout, so
+// that fragment ks is the operand read k_off(k_base, ks) of a K stage.  Loaded
+// straight into fragments, each instruction would read 32 bytes of each of 32
+// rows, and a workgroup's 64 such loads kept its vector-memory path busy for
+// ~4500 of a work item's ~12,000 prologue cycles.  Work item start to stage loop,
+// before and after: key-split pairs 11.9k -> 7.0k ticks (H=56 S=10000), 128-row
+// pairs 13.3k -> 9.3k, dense 11.5k -> 10.9k (its 64 KiB of query rows per item
+// come from HBM and set the pace), 8.5k -> 6.1k where they come from L2.
+// Rows past Sq repeat the last row (64-bit addresses: no limit on the stride);
+// what becomes of them is never stored.
+template <class L>
+struct QTile {
+  static_assert(L::kKRow == 256 && L::kKSlots == 16, "one K row per query row");
+  static constexpr int kInst = 8;
+  // Instructions I0 .. I1-1 of the 8.
+  template <int I0, int I1>
+  __device__ __forceinline__ static void issue(const uint16_t *Qb, int64_t qss, int q0, int Sq, int lane,
+                                               uint16_t *tile) {
+    uint32_t m0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_address(tile)) + 1024u * I0;
+#pragma unroll
+    for (int i = I0; i < I1; ++i) {
+      const int r = 4 * i + (lane >> 4);
+      const int row = q0 + r < Sq ? q0 + r : Sq - 1;
+      global_load_lds_b128(Qb + (int64_t)row * qss + 8 * L::k_chunk(r, lane & 15), m0);
+      m0 = opaque_sadd<1024u>(m0);
+    }
+  }
+  __device__ __forceinline__ static void read(u32x4 (&qf)[8], const uint16_t *tile, int k_rd) {
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks)
+      qf[ks] = *(const u32x4 *)(reinterpret_cast<const char *>(tile) + L::k_off(k_rd, ks));
+  }
 };
 
 // One work item of attn_fwd_pingpong_kernel: a 256-row query tile, a key
@@ -775,6 +811,28 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
     }
   }
   const int qrow = kSparse ? qb * QB + rq * 32 + l32 : qt * 256 + wave * 32 + l32;
+  // The wave's query rows are on their way before anything else is waited for.
+  // Dense: a tile per wave.  Sparse: in buffers that the prologue fills late or
+  // not at all: 128-row blocks, a tile per wave in the group's K(1) and V(1)
+  // buffers; 64-row blocks, one tile per 32-row slice in its V(1) buffer, each of
+  // the slice's two waves fetching half.
+  uint16_t *qtile;
+  if constexpr (!kSparse) {
+    qtile = lds.q + wave_u * 32 * kD;
+  } else if constexpr (kKeySplit) {
+    qtile = vbuf[1] + rq * 32 * kD;
+  } else {
+    qtile = (rq < 2 ? kbuf[1] : vbuf[1]) + (rq & 1) * 32 * kD;
+  }
+  {
+    const int q0 = __builtin_amdgcn_readfirstlane(qrow - l32);
+    if constexpr (kKeySplit) {
+      if (kh == 0) QTile<L>::template issue<0, 4>(Qb, a.qss, q0, a.Sq, lane, qtile);
+      else QTile<L>::template issue<4, 8>(Qb, a.qss, q0, a.Sq, lane, qtile);
+    } else {
+      QTile<L>::template issue<0, 8>(Qb, a.qss, q0, a.Sq, lane, qtile);
+    }
+  }
   // Sparse: this group's stage count and LUT row; both groups run the longer
   // of the two lists.  A piece of a split pair runs stages [gj0, gj0 + ngrp)
   // of the group's list.
@@ -897,17 +955,6 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
     return;
   }
 
-  // Global loads: as flat loads they would also count as LDS/scalar accesses
-  // and hold up the next wait for those.
-  u32x4 qf[8];
-  if (qrow < a.Sq) {
-    const uint16_t *p = Qb + (int64_t)qrow * a.qss + 8 * g;
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) qf[ks] = *(const __attribute__((address_space(1))) u32x4 *)(p + ks * 16);
-  } else {
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) qf[ks] = u32x4{0, 0, 0, 0};
-  }
   f32x16 o[4];
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) o[dt] = f32x16{0.f};
@@ -985,14 +1032,15 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
     vcur.init(Vb, a.vss, (j0 + 1) * BN, key_end);
   }
 
-  // Prologue, all waves in step: K(0), V(0), K(1) in; S(0); P(0).  Dense:
-  // group B fetches the K stages, group A the V stage.
+  // Prologue, all waves in step: Q, K(0), V(0), K(1) in; S(0); P(0).  Dense:
+  // group B fetches the K stages, group A the V stage.  128-row blocks: K(1)
+  // lands during S(0), once the query tiles are read out of its place.
   const int pkey0 = pro_key(0), pkey1 = pro_key(1);
   const uint32_t pmask0 = kTileMask ? (uint32_t)pro_entry(0) & 0xffu : 0u;
   if constexpr (kSparse) {
     kdma.issue(Kb, a.kss, pkey0, a.Skv, kdst(kbuf[0]));
     vdma.issue(Vb, a.vss, pkey0, a.Skv, vdst(vbuf[0]));
-    kdma.issue(Kb, a.kss, pkey1, a.Skv, kdst(kbuf[1]));
+    if constexpr (kKeySplit) kdma.issue(Kb, a.kss, pkey1, a.Skv, kdst(kbuf[1]));
   } else if (lead) {
     vdma.issue(Vb, a.vss, pkey0, a.Skv, vbuf[0]);
   } else {
@@ -1001,12 +1049,21 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
   }
   wait_vmem_all();
   __syncthreads();
+  u32x4 qf[8];
+  QTile<L>::read(qf, qtile, L::k_base(l32, g));
+  if constexpr (kSparse && !kKeySplit) {
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) pin(qf[ks]);
+    __syncthreads();  // every query tile is read: K(1) may land
+    kdma.issue(Kb, a.kss, pkey1, a.Skv, kbuf[1]);
+  }
   f32x16 s[WS];
   u32x4 pf[2 * WS];
   score_tile<L, WS>(kbuf[0], qf, k_rd, s);
   if constexpr (kTileMask) apply_tile_mask<WS>(s, pmask0, rq, l32);
   softmax_stage<WS>(s, pkey0 + (kTileMask ? 0 : 32 * kh), a.Skv, g, a.sl2, m, lsum, o, pf);
-  __syncthreads();  // kbuf[0] is free for K(2)
+  if constexpr (kSparse && !kKeySplit) wait_vmem_all();
+  __syncthreads();  // kbuf[0] is free for K(2); key-split: the query tiles for V(1)
 
   // Dense, stage j's fetch from the stream cursors: group A's V(j+1) into
   // vbuf[(j+1)&1], group B's K(j+2) into kbuf[j&1].
@@ -1205,16 +1262,12 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
   }
   pc.loop_end();
   // Sparse: group B's last stage issued loads (of nothing: keys past its
-  // list) into group B's K/V buffers that may still be in flight.  The
-  // key-split exchange below writes those buffers from other waves, so there
-  // every wave waits for its loads and a barrier follows.  Otherwise nothing
-  // touches group B's buffers before this wave's next fetch into them, which
-  // lands after these (a wave's loads complete in order), and the kernel
-  // waits for them before it exits.
-  if constexpr (kKeySplit) {
-    wait_vmem_all();
-    __syncthreads();
-  }
+  // list) into group B's K/V buffers that may still be in flight.  They land
+  // before the wave goes on: the next work item's query tiles, fetched by other
+  // waves than these, use the same buffers.  The key-split exchange below
+  // writes them too, from other waves, so there a barrier follows.
+  if constexpr (kSparse) wait_vmem_all();
+  if constexpr (kKeySplit) __syncthreads();
 
   if constexpr (kKeySplit) {
     // Every LDS read and write of the stages is complete (the barrier
@@ -1277,8 +1330,7 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
   // read back a chunk per lane, every store writes 4 whole rows.  The tile is
   // free: key-split, the wave's own exchange slot, which it has read;
   // otherwise a quarter of group A's K or V buffers, whose fetches all
-  // completed before the loop's last barrier (group B's last loads, still in
-  // flight for other waves, only touch group B's buffers).
+  // completed before the loop's last barrier.
   {
     uint8_t *tile;
     if constexpr (kKeySplit) {

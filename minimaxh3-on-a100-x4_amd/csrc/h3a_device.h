@@ -97,6 +97,11 @@ __device__ __forceinline__ void buffer_load_lds_b128(u32x4 desc, uint32_t byte_o
                : "memory");
 }
 
+// The same from a 64-bit address per lane, with no range check.
+__device__ __forceinline__ void global_load_lds_b128(const void *p, uint32_t m0) {
+  asm volatile("global_load_lds_dwordx4 %0, off" ::"v"(p), "{m0}"(m0) : "memory");
+}
+
 // LDS byte address of a pointer into a __shared__ array.
 __device__ __forceinline__ uint32_t lds_address(const void *p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
