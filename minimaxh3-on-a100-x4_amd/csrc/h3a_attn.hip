@@ -27,6 +27,8 @@
 //    a stale reference max and takes a row max only when a stage's p sum
 //    overflows its bound.  A split tail cuts the last, partly filled round of
 //    query tiles into key ranges merged by split_combine_kernel.
+//    Launches of few tiles take shorter ones, 128 or 64 rows, whose two groups
+//    share the keys of one query block (kHalves; the rule is plan_attn_split's).
 //  * Block-sparse (attn_fwd_pingpong_kernel with kSparse): the ping-pong
 //    over a pair of query blocks, one per group, each with its own LUT row
 //    and K/V stream fetched by LDS DMA into swizzled rows; a group issues its
@@ -41,6 +43,7 @@
 //    FMA; workgroup ids are remapped XCD-aware (xcd_remap).
 #include <atomic>
 #include <climits>
+#include <cstddef>
 #include <type_traits>
 
 #include "h3a_device.h"
@@ -736,7 +739,13 @@ struct QTile {
 // range of a split tile, or (sparse) a pair of query blocks or a piece of one.
 // `remapped`: the item number is already XCD-aware (taken from the queues),
 // so whole tiles are not remapped.
-template <class L, int NSUB, bool kSparse, bool kKeySplit, bool kWideKV, bool kTileMask>
+//
+// kHalves (with kSparse): dense attention on a short tile, 128 query rows or
+// (kKeySplit) 64.  Both groups take the same rows, group x the key stages
+// s0 + x, s0 + x + 2, ... of the range, so that with kKeySplit every 32-row slice
+// is spread over four waves, otherwise over two; after the loop they exchange
+// their parts through LDS, each wave merging and storing its share of the dims.
+template <class L, int NSUB, bool kSparse, bool kKeySplit, bool kWideKV, bool kTileMask, bool kHalves>
 __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item, const bool remapped,
                                               PingPongLds<L, NSUB, kSparse> &lds, PhaseClock &pc) {
   constexpr int NW = 8;
@@ -747,6 +756,7 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
   static_assert(!kSparse || BN == kBN, "block-sparse stages are 64 keys");
   static_assert(!kKeySplit || (kSparse && NSUB == 2), "key-split pairs are block-sparse, 64-key stages");
   static_assert(!kTileMask || kKeySplit, "tile masks run on the key-split pairs");
+  static_assert(!kHalves || (kSparse && !kTileMask), "key halves run on the pairs kernels");
   auto &kbuf_all = lds.k;
   auto &vbuf_all = lds.v;
 
@@ -784,7 +794,8 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
     niter = (int)((int64_t)nstages * (p + 1) / a.split_pieces) - j0;  // >= 1
   }
   // Sparse: a.nqt counts query sub-blocks of QB rows and w runs over (b, h, pair).
-  const int nw_bh = kSparse ? (a.nqt + 1) / 2 : a.nqt;
+  // (kHalves: over tiles of QB rows.)
+  const int nw_bh = kSparse && !kHalves ? (a.nqt + 1) / 2 : a.nqt;
   const int qt = w % nw_bh, bh = w / nw_bh;
   const int h = bh % a.H, b = bh / a.H;
   const uint16_t *Qb = a.q + b * a.qsb + h * a.qsh;
@@ -798,7 +809,7 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
   // Sparse: the pair's query sub-blocks, this group's (qb) and the other
   // group's (qo): 2qt and 2qt+1, or (tile path) the pair map's, clamped into
   // [0, nqt] (sub-block nqt is past the end: no rows, no stages).
-  int qb = 2 * qt + grp, qo = 2 * qt + 1 - grp;
+  int qb = kHalves ? qt : 2 * qt + grp, qo = kHalves ? qt : 2 * qt + 1 - grp;
   if constexpr (kTileMask) {
     if (a.pair_map) {
       typedef const __attribute__((address_space(4))) int32_t *ConstInts;
@@ -844,7 +855,12 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
   // own column: its fetch, scores and mask).  ntile is the row's entry count.
   int ntile = 0;
   const uint32_t smag = stage_magic(a.sub);  // block_of_stage_magic(t, smag) = t / a.sub
-  if constexpr (kSparse) {
+  if constexpr (kHalves) {
+    j0 = split_part < 0 ? 0 : (int)((int64_t)nstages * split_part / a.split_pieces);
+    const int len = (split_part < 0 ? nstages : (int)((int64_t)nstages * (split_part + 1) / a.split_pieces)) - j0;
+    ngrp = (len + 1 - grp) / 2;  // this group's stages: j0 + grp + 2j
+    niter = (len + 1) / 2;       // >= 1
+  } else if constexpr (kSparse) {
     // Query sub-block qb reads LUT row qb / a.qmul (blk_q = 256: the two
     // 128-row blocks of a pair share one row; blk_q = 192: three 64-row ones).
     // The counts and the LUT are read through the constant address space:
@@ -894,7 +910,7 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
   // group's part of the row (entry 0 for an empty list, whose keys are all
   // Skv whatever the entry).
   auto lut_entry = [&](int j) __attribute__((always_inline)) -> int {
-    if constexpr (kSparse) {
+    if constexpr (kSparse && !kHalves) {
       const __attribute__((address_space(4))) int32_t *row =
           (const __attribute__((address_space(4))) int32_t *)lut_row;
       const int jc = j < ngrp ? j : ngrp - 1;
@@ -913,7 +929,9 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
   // entry negative, so it still names no key block.  Past the row's entries
   // (the last stage can hold one column) the key is Skv.
   auto key_of_entry = [&](int j, int e) __attribute__((always_inline)) -> int {
-    if constexpr (kSparse) {
+    if constexpr (kHalves) {
+      return j < ngrp ? (j0 + grp + 2 * j) * BN : a.Skv;
+    } else if constexpr (kSparse) {
       const int kb = kTileMask ? (e >> 8) : e;
       // Two equivalent forms; each measured faster in one kernel (the
       // arithmetic one +0.5 % in the 128-row pairs, the select one +0.6 % in
@@ -929,11 +947,11 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
   auto key_base = [&](int j) __attribute__((always_inline)) -> int { return key_of_entry(j, lut_entry(j)); };
   // The same for the prologue's stages 0-3, from the entries loaded up front.
   auto pro_entry = [&](int j) __attribute__((always_inline)) -> int {
-    if constexpr (kSparse) return split_part < 0 ? e_pre[j] : lut_entry(j);
+    if constexpr (kSparse && !kHalves) return split_part < 0 ? e_pre[j] : lut_entry(j);
     else return 0;
   };
   auto pro_key = [&](int j) __attribute__((always_inline)) -> int { return key_of_entry(j, pro_entry(j)); };
-  if (kSparse && niter == 0) {
+  if (kSparse && !kHalves && niter == 0) {
     // Neither query block of the pair keeps a key block (in this piece): O = 0,
     // or an empty partial result (m = -inf, l = 0, O = 0).
     if (piece >= 0) {
@@ -1267,7 +1285,76 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
   // waves than these, use the same buffers.  The key-split exchange below
   // writes them too, from other waves, so there a barrier follows.
   if constexpr (kSparse) wait_vmem_all();
-  if constexpr (kKeySplit) __syncthreads();
+  if constexpr (kKeySplit || kHalves) __syncthreads();
+
+  if constexpr (kHalves) {
+    // The parts of a 32-row slice: wave u of NP holds (O, m, l) over its keys.
+    // Wave u merges and stores dims 32*KD*u .. of the slice, so it leaves the
+    // others' dims in LDS (every K/V read is complete: the barrier above), a
+    // 4 KiB slot per (slice, wave, 32 dims), and its m and l in the first slot
+    // of its own dims.
+    constexpr int NP = kKeySplit ? 4 : 2, KD = 4 / NP;
+    using Lds = PingPongLds<L, NSUB, kSparse>;
+    static_assert(sizeof(lds.k) + sizeof(lds.v) == 8 * 4 * 4096 && offsetof(Lds, v) == sizeof(lds.k),
+                  "the K and V buffers are 8 waves x 4 slots, contiguous");
+    float *xch = reinterpret_cast<float *>(&kbuf_all[0][0][0]);
+    const int u = kKeySplit ? 2 * grp + kh : grp;
+    auto slot = [&](int wv, int dt) __attribute__((always_inline)) { return xch + ((rq * NP + wv) * 4 + dt) * 1024; };
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) {
+      if (dt / KD == u) continue;
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr)
+        *(float4 *)(slot(u, dt) + rr * 256 + lane * 4) =
+            float4{o[dt][4 * rr], o[dt][4 * rr + 1], o[dt][4 * rr + 2], o[dt][4 * rr + 3]};
+    }
+    *(float2 *)(slot(u, KD * u) + lane * 2) = float2{m, lsum};
+    __syncthreads();
+    float2 ml[NP];
+    float mn = kNegInf, lall = 0.f, w8[NP];
+#pragma unroll
+    for (int v = 0; v < NP; ++v) {
+      ml[v] = *(const float2 *)(slot(v, KD * v) + lane * 2);
+      mn = fmaxf(mn, ml[v].x);
+    }
+#pragma unroll
+    for (int v = 0; v < NP; ++v) {
+      w8[v] = ml[v].x == kNegInf ? 0.f : fast_exp2(ml[v].x - mn);
+      lall = fmaf(ml[v].y, w8[v], lall);
+    }
+    const float ltot = half_swap_sum(lall);
+    const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
+    const int trow = rq * 32 + l32;  // row of the tile
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) {
+      if (dt / KD != u) continue;
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) {
+        float4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int v = 0; v < NP; ++v) {
+          const float4 p = v == u ? float4{o[dt][4 * rr], o[dt][4 * rr + 1], o[dt][4 * rr + 2], o[dt][4 * rr + 3]}
+                                  : *(const float4 *)(slot(v, dt) + rr * 256 + lane * 4);
+          acc.x = fmaf(w8[v], p.x, acc.x);
+          acc.y = fmaf(w8[v], p.y, acc.y);
+          acc.z = fmaf(w8[v], p.z, acc.z);
+          acc.w = fmaf(w8[v], p.w, acc.w);
+        }
+        const int dim = dt * 32 + 8 * rr + 4 * g;
+        if (piece >= 0) {
+          *(float4 *)(a.ws + ((int64_t)piece * QB + trow) * kD + dim) = acc;
+        } else if (qrow < a.Sq) {
+          *(u32x2 *)(Ob + (int64_t)qrow * a.oss + dim) =
+              u32x2{pack_bf16x2(acc.x * inv, acc.y * inv), pack_bf16x2(acc.z * inv, acc.w * inv)};
+        }
+      }
+    }
+    if (piece >= 0 && u == 0 && g == 0)
+      *(float2 *)(a.ws + (int64_t)(a.total - a.split_first) * QB * kD + ((int64_t)piece * QB + trow) * 2) =
+          float2{mn, ltot};
+    pc.finish(wave, lane);
+    return;
+  }
 
   if constexpr (kKeySplit) {
     // Every LDS read and write of the stages is complete (the barrier
@@ -1368,7 +1455,7 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
 }
 
 template <class L, int NSUB, bool kSparse = false, bool kKeySplit = false, bool kWideKV = false,
-          bool kTileMask = false>
+          bool kTileMask = false, bool kHalves = false>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 attn_fwd_pingpong_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(16))) PingPongLds<L, NSUB, kSparse> lds;
@@ -1410,7 +1497,7 @@ attn_fwd_pingpong_kernel(AttnArgs a) {
       if (item < 0) break;
     }
     pc.begin(blockIdx.x == 0);
-    pingpong_item<L, NSUB, kSparse, kKeySplit, kWideKV, kTileMask>(args, item, args.sched != nullptr, lds, pc);
+    pingpong_item<L, NSUB, kSparse, kKeySplit, kWideKV, kTileMask, kHalves>(args, item, args.sched != nullptr, lds, pc);
     KernargPtr kq = (KernargPtr)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(kq));
     if (!kq->sched) break;
@@ -1428,38 +1515,59 @@ __global__ void __launch_bounds__(256) sched_clear_kernel(int *sched) {
 
 // Merge the key-range pieces of the split tiles:
 //   O = sum_p 2^(m_p - M) O_p / sum_p 2^(m_p - M) l_p,  M = max_p m_p.
-// One thread per (split tile, row, 4 dims); 8 rows per 256-thread block.
+// One thread per (split tile, row, 4 dims); 8 rows per 256-thread block; tiles of
+// a.tile_rows rows.  A thread's loads depend on nothing, so kCombineUnroll pieces
+// are in flight at a time; one after another they were a chain of P round trips
+// (8.6 us for 32 tiles of 256 rows in 8 pieces, 35 MB).
+constexpr int kCombineUnroll = 4;
 __global__ void __launch_bounds__(256) split_combine_kernel(AttnArgs a) {
   const int ntiles = (a.total - a.split_first) / a.split_pieces;
+  const int R = a.tile_rows;
   const int64_t item = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 5);  // (split tile, row)
-  if (item >= (int64_t)ntiles * 256) return;
-  const int t = (int)(item / 256), row = (int)(item % 256), d = 4 * (threadIdx.x & 31);
+  if (item >= (int64_t)ntiles * R) return;
+  const int t = (int)(item / R), row = (int)(item % R), d = 4 * (threadIdx.x & 31);
   const int tile = a.split_first + t;
   const int tiles_bh = a.lut ? (a.nqt + 1) / 2 : a.nqt;  // sparse: pairs of 128-row blocks
   const int qt = tile % tiles_bh, bh = tile / tiles_bh;
   const int h = bh % a.H, b = bh / a.H;
-  const int qrow = qt * 256 + row;
+  const int qrow = qt * R + row;
   if (qrow >= a.Sq) return;
   const int P = a.split_pieces;
-  const float *ml = a.ws + (int64_t)(a.total - a.split_first) * 256 * kD;
+  const float *ml = a.ws + (int64_t)(a.total - a.split_first) * R * kD + ((int64_t)t * P * R + row) * 2;
+  const float *po = a.ws + ((int64_t)t * P * R + row) * kD + d;
   float M = kNegInf;
-  for (int p = 0; p < P; ++p) M = fmaxf(M, ml[((int64_t)(t * P + p) * 256 + row) * 2]);
+  for (int p0 = 0; p0 < P; p0 += 2 * kCombineUnroll) {
+    float mv[2 * kCombineUnroll];
+#pragma unroll
+    for (int u = 0; u < 2 * kCombineUnroll; ++u) mv[u] = ml[(int64_t)(p0 + u < P ? p0 + u : 0) * R * 2];
+#pragma unroll
+    for (int u = 0; u < 2 * kCombineUnroll; ++u) M = fmaxf(M, mv[u]);
+  }
   float4 acc = {0.f, 0.f, 0.f, 0.f};
   float L = 0.f;
-  for (int p = 0; p < P; ++p) {
-    const int64_t pr = (int64_t)(t * P + p) * 256 + row;
-    const float mp = ml[pr * 2], lp = ml[pr * 2 + 1];
-    const float wgt = (mp == kNegInf) ? 0.f : fast_exp2(mp - M);
-    const float4 op = *(const float4 *)(a.ws + pr * kD + d);
-    acc.x = fmaf(wgt, op.x, acc.x);
-    acc.y = fmaf(wgt, op.y, acc.y);
-    acc.z = fmaf(wgt, op.z, acc.z);
-    acc.w = fmaf(wgt, op.w, acc.w);
-    L = fmaf(wgt, lp, L);
+  for (int p0 = 0; p0 < P; p0 += kCombineUnroll) {
+    float2 mv[kCombineUnroll];
+    float4 ov[kCombineUnroll];
+#pragma unroll
+    for (int u = 0; u < kCombineUnroll; ++u) {
+      const int64_t pr = (int64_t)(p0 + u < P ? p0 + u : 0) * R;
+      mv[u] = *(const float2 *)(ml + pr * 2);
+      ov[u] = *(const float4 *)(po + pr * kD);
+    }
+#pragma unroll
+    for (int u = 0; u < kCombineUnroll; ++u) {
+      if (p0 + u >= P) break;
+      const float wgt = (mv[u].x == kNegInf) ? 0.f : fast_exp2(mv[u].x - M);
+      acc.x = fmaf(wgt, ov[u].x, acc.x);
+      acc.y = fmaf(wgt, ov[u].y, acc.y);
+      acc.z = fmaf(wgt, ov[u].z, acc.z);
+      acc.w = fmaf(wgt, ov[u].w, acc.w);
+      L = fmaf(wgt, mv[u].y, L);
+    }
   }
   const float inv = L > 0.f ? 1.f / L : 0.f;
-  uint16_t *po = a.o + b * a.osb + h * a.osh + (int64_t)qrow * a.oss + d;
-  *(u32x2 *)po = u32x2{pack_bf16x2(acc.x * inv, acc.y * inv), pack_bf16x2(acc.z * inv, acc.w * inv)};
+  uint16_t *out = a.o + b * a.osb + h * a.osh + (int64_t)qrow * a.oss + d;
+  *(u32x2 *)out = u32x2{pack_bf16x2(acc.x * inv, acc.y * inv), pack_bf16x2(acc.z * inv, acc.w * inv)};
 }
 
 // ---------------------------------------------------------------------------
@@ -1668,7 +1776,9 @@ static int device_cu_count(int *cus_out) {
 // tiles run on a persistent grid fed by the per-XCD queues (take_item): the
 // XCDs' clocks differ under full load by up to ~5 %, and with a static
 // deal the fastest XCD idles while the slowest finishes its share.
-static int plan_tiles(int64_t tiles, int stages, bool splittable, bool queued, SplitPlan *plan) {
+// `max_pieces` bounds the ranges per tile; `rows` is the tile height.
+static int plan_tiles(int64_t tiles, int stages, bool splittable, bool queued, SplitPlan *plan,
+                      int max_pieces = INT_MAX, int rows = 256) {
   constexpr int kMinSplitStages = 4;
   constexpr int64_t kQueuedRounds = 4;
   int cus = 0;
@@ -1679,14 +1789,15 @@ static int plan_tiles(int64_t tiles, int stages, bool splittable, bool queued, S
   if (splittable && r > 0) {
     const int64_t by_cus = cus / r, by_len = stages / kMinSplitStages;
     pieces = (int)(by_cus < by_len ? by_cus : by_len);
+    if (pieces > max_pieces) pieces = max_pieces;
   }
   const int clamped = (int)(tiles > INT_MAX ? INT_MAX : tiles);
-  *plan = SplitPlan{clamped, clamped, 1, 0, false, 0};
+  *plan = SplitPlan{clamped, clamped, 1, 0, false, 0, false, 256};
   if (tiles > INT_MAX) return H3A_OK;
   if (pieces >= 2) {
     plan->first = (int)(tiles - r);
     plan->pieces = pieces;
-    plan->bytes = (size_t)r * pieces * 256 * (kD + 2) * sizeof(float);
+    plan->bytes = (size_t)r * pieces * rows * (kD + 2) * sizeof(float);
   }
   if (queued && tiles >= kQueuedRounds * cus) {
     plan->dynamic = true;
@@ -1696,8 +1807,77 @@ static int plan_tiles(int64_t tiles, int stages, bool splittable, bool queued, S
   return H3A_OK;
 }
 
+// Dense tile heights and what they cost in shader cycles (phase profile, whole
+// chip busy): a pair of 64-key stages, and an item's prologue and epilogue.
+// 256 rows share one K/V stream and run 4-5 % more rows per cycle than two
+// 128-row tiles, whose groups each fetch their own; 64 rows cost 38 % more per
+// row again.  But a launch of few tiles leaves CUs idle or cuts them into many
+// key ranges, each with its own prologue and 520 bytes of partial sums a row: at
+// 128 or 64 rows there are more, shorter items instead.
+struct DenseForm {
+  int rows, pair_cycles, item_cycles;
+};
+constexpr DenseForm kDenseForms[] = {{256, 2 * 2567, 13000}, {128, 2860, 12000}, {64, 1980, 10000}};
+// The combine: a launch's latency, and its reads and the partials' writes at
+// about 1000 cycles a megabyte (35 MB: 8.6 us to read, about 7 to write).
+constexpr int kCombineCycles = 9000, kCombineCyclesPerMB = 1000;
+
+// The form and the number of key ranges of the tail with the least estimated
+// time: whole rounds of tiles, then the last round's r tiles in P ranges each
+// (P = 1 .. CUs / r with at least kMinSplitStages stages per range; at least 2
+// after a whole round, where the combine is a small part of the launch).  Measured per call, 256 / 128 / 64 rows (one
+// card, graph replay): H=2 S=300 11.0 / 11.5 / 8.6 us; H=4 S=2048 26.5 / 26.8 /
+// 18.8; H=14 S=1000 23.1 / 18.8 / 14.0; H=28 S=700 18.3 / 17.0 / 24.3; H=4 S=8000
+// 125.3 / 120.7 / 137.0; H=14 S=3000 64.5 / 77.5 / 80.5; H=56 S=2000 108.6 / 130.5 /
+// 148.7; the choice is within 0.6 us of the least in each.
 int plan_attn_split(int B, int H, int Sq, int Skv, SplitPlan *plan) {
-  return plan_tiles((int64_t)B * H * ((Sq + 255) / 256), (Skv + kBN - 1) / kBN, true, true, plan);
+  int cus = 0;
+  int rc = device_cu_count(&cus);
+  if (rc) return rc;
+  const int stages = (Skv + kBN - 1) / kBN;
+  int64_t best = -1;
+  bool splits = false;
+  for (const DenseForm &f : kDenseForms) {
+    const int64_t tiles = (int64_t)B * H * (((int64_t)Sq + f.rows - 1) / f.rows);
+    if (tiles > INT_MAX && f.rows != 256) continue;
+    SplitPlan p;
+    rc = plan_tiles(tiles, stages, true, true, &p);
+    if (rc) return rc;
+    // Cycles of a round of items of n stages on `busy` CUs, in cycles of a full
+    // chip's clock: the power limit holds 256 busy CUs at about 1.7 GHz, and
+    // fewer run faster, up to 2.35 GHz (72 % of the time) at 184 CUs and less.
+    auto pass = [&](int n, int64_t busy) -> int64_t {
+      const int64_t cycles = (int64_t)(n + 1) / 2 * f.pair_cycles + f.item_cycles;
+      const int64_t pct = 100 * busy / cus;
+      return cycles * (pct < 72 ? 72 : pct) / 100;
+    };
+    const int64_t r = tiles % cus, full = tiles / cus * pass(stages, cus);
+    int64_t cost = full + (r ? pass(stages, r) : 0);
+    splits = splits || p.pieces >= 2;
+    if (p.pieces >= 2) {
+      int pieces = 1;
+      for (int n = 2; n <= p.pieces; ++n) {
+        const int64_t kb = r * n * f.rows * (int64_t)((kD + 2) * sizeof(float)) / 1024;
+        const int64_t c =
+            full + pass((stages + n - 1) / n, r * n) + kCombineCycles + kb * kCombineCyclesPerMB / 1024;
+        if (c < cost || (n == 2 && tiles > cus)) {
+          cost = c;
+          pieces = n;
+        }
+      }
+      rc = plan_tiles(tiles, stages, true, true, &p, pieces, f.rows);
+      if (rc) return rc;
+    }
+    p.rows = f.rows;
+    if (best < 0 || cost < best) {
+      best = cost;
+      *plan = p;
+    }
+  }
+  // A launch that some form would split asks for a workspace, so that a caller
+  // prepared for one does not depend on the form.
+  if (splits && plan->bytes == 0) plan->bytes = 256;
+  return H3A_OK;
 }
 
 // The longest list a query block can hold (max_k_blocks key blocks) stands in
@@ -1731,9 +1911,10 @@ int plan_attn_sparse_tiles(int B, int H, int Sq, int max_tiles, SplitPlan *plan)
 // Workgroups of a persistent launch of `kernel` (512 threads): every CU
 // filled to its occupancy, cached per device.
 // `slot` names the kernel in the cache (0 dense, 1 sparse pairs, 2 sparse
-// key-split, 3 sparse key-split over tile masks).
+// key-split, 3 sparse key-split over tile masks, 4 and 5 dense in 128- and
+// 64-row tiles).
 static int persistent_grid(const void *kernel, int slot, int *grid) {
-  static std::atomic<int> grid_cache[64][4];
+  static std::atomic<int> grid_cache[64][6];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return fail(H3A_ERR_HIP, "hipGetDevice failed");
   std::atomic<int> *cached = (dev >= 0 && dev < 64) ? &grid_cache[dev][slot] : nullptr;
@@ -1751,9 +1932,28 @@ static int persistent_grid(const void *kernel, int slot, int *grid) {
   return H3A_OK;
 }
 
+typedef void (*PingPongKernel)(AttnArgs);
+// Stage offsets from the (b,h) slice base could pass 2^32 bytes (see kWideKV).
+static bool wide_kv(const AttnArgs &a) {
+  const int64_t stride = a.kss > a.vss ? a.kss : a.vss;
+  return ((int64_t)a.Skv + 64) * stride * 2 >= ((int64_t)1 << 32);
+}
+
+static PingPongKernel dense_pingpong_kernel(const AttnArgs &a, int rows) {
+  const bool wide = wide_kv(a);
+  if (rows == 128)
+    return wide ? attn_fwd_pingpong_kernel<SwzLayout, kStageSub, true, false, true, false, true>
+                : attn_fwd_pingpong_kernel<SwzLayout, kStageSub, true, false, false, false, true>;
+  if (rows == 64)
+    return wide ? attn_fwd_pingpong_kernel<SwzLayout, kStageSub, true, true, true, false, true>
+                : attn_fwd_pingpong_kernel<SwzLayout, kStageSub, true, true, false, false, true>;
+  return attn_fwd_pingpong_kernel<SwzLayout, kStageSub>;
+}
+
 int launch_attn_dense_split(AttnArgs a, const SplitPlan &plan, void *ws, hipStream_t s) {
-  if (plan.pieces < 2 && !plan.dynamic) return launch_attn_dense(a, s);
-  a.nqt = (a.Sq + 255) / 256;
+  if (plan.pieces < 2 && !plan.dynamic && plan.rows == 256) return launch_attn_dense(a, s);
+  a.nqt = (int)(((int64_t)a.Sq + plan.rows - 1) / plan.rows);
+  a.tile_rows = plan.rows;
   if (plan.pieces >= 2) {
     a.split_first = plan.first;
     a.split_pieces = plan.pieces;
@@ -1762,10 +1962,11 @@ int launch_attn_dense_split(AttnArgs a, const SplitPlan &plan, void *ws, hipStre
   const int64_t total = (int64_t)plan.first + (int64_t)(plan.tiles - plan.first) * plan.pieces;
   if (total > INT_MAX) return fail(H3A_ERR_INVALID_ARG, "too many work items (%lld)", (long long)total);
   a.total = (int)total;
-  auto kernel = attn_fwd_pingpong_kernel<SwzLayout, kStageSub>;
+  const PingPongKernel kernel = dense_pingpong_kernel(a, plan.rows);
   int grid = a.total, rc;
   if (plan.dynamic) {
-    rc = persistent_grid(reinterpret_cast<const void *>(kernel), 0, &grid);
+    rc = persistent_grid(reinterpret_cast<const void *>(kernel), plan.rows == 256 ? 0 : (plan.rows == 128 ? 4 : 5),
+                         &grid);
     if (rc) return rc;
     if (grid > a.total) grid = a.total;
     a.sched = reinterpret_cast<int *>(static_cast<char *>(ws) + plan.sched_off);
@@ -1776,7 +1977,7 @@ int launch_attn_dense_split(AttnArgs a, const SplitPlan &plan, void *ws, hipStre
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(512), 0, s, a);
   rc = check_launch("attn_fwd_pingpong_kernel<split>");
   if (rc || plan.pieces < 2) return rc;
-  const int64_t rows = (int64_t)(plan.tiles - plan.first) * 256;
+  const int64_t rows = (int64_t)(plan.tiles - plan.first) * plan.rows;
   hipLaunchKernelGGL(split_combine_kernel, dim3((unsigned)((rows + 7) / 8)), dim3(256), 0, s, a);
   return check_launch("split_combine_kernel");
 }
@@ -1785,10 +1986,8 @@ int launch_attn_dense_split(AttnArgs a, const SplitPlan &plan, void *ws, hipStre
 // `tiles`: the key-split pairs over a tile LUT with sub-block masks); the
 // wide-K/V instantiation when stage offsets from the (b,h) slice base could
 // pass 2^32 bytes (see kWideKV).
-typedef void (*PingPongKernel)(AttnArgs);
 static PingPongKernel sparse_pingpong_kernel(const AttnArgs &a, int rows, bool tiles) {
-  const int64_t stride = a.kss > a.vss ? a.kss : a.vss;
-  const bool wide = ((int64_t)a.Skv + 64) * stride * 2 >= ((int64_t)1 << 32);
+  const bool wide = wide_kv(a);
   if (tiles)
     return wide ? attn_fwd_pingpong_kernel<SwzLayout, kStageSub, true, true, true, true>
                 : attn_fwd_pingpong_kernel<SwzLayout, kStageSub, true, true, false, true>;

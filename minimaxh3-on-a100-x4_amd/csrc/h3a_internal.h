@@ -44,6 +44,7 @@ struct AttnArgs {
   // cut into split_pieces key ranges whose partial results go to ws
   int split_first;
   int split_pieces;
+  int tile_rows;  // rows of a split tile (256; dense also 128 or 64)
   float *ws;
   // dynamic dispatch (persistent grid, per-XCD work queues): the queues'
   // counters, zeroed before the launch; null for one work item per workgroup
@@ -79,6 +80,7 @@ struct SplitPlan {
   bool dynamic; // persistent grid with per-XCD work queues
   size_t sched_off;  // byte offset of the queue counters in the workspace
   bool pair_map;     // tile path: sub-blocks paired by stage count (map at offset 0)
+  int rows;          // dense: tile height (256, 128 or 64)
 };
 
 // Launchers implemented in h3a_attn.hip / h3a_prologue.hip.

@@ -101,10 +101,10 @@ def attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float | N
     args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
             B, H, Sq, Skv, D, _bhs(q), _bhs(k), _bhs(v), _bhs(out), sc)
     with torch.cuda.device(q.device):
-        nbytes = attn_workspace_bytes(B, H, Sq, Skv, D) if split_tail else 0
-        if nbytes:
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
-            rc = lib().h3a_attn_fwd_ws(*args, ws.data_ptr(), nbytes, _stream(q))
+        if split_tail:
+            nbytes = attn_workspace_bytes(B, H, Sq, Skv, D)
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+            rc = lib().h3a_attn_fwd_ws(*args, ws.data_ptr() if nbytes else None, nbytes, _stream(q))
             check("h3a_attn_fwd_ws", rc)
         else:
             rc = lib().h3a_attn_fwd(*args, _stream(q))

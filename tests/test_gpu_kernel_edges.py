@@ -1,9 +1,12 @@
 """GPU: each kernel form at the sizes where its dispatch or its tiling can go wrong (tile edges,
 remainders, the smallest of its range), against the oracle or the form it must equal bit for bit."""
+import numpy as np
 import pytest
 import torch
 
 import h3attn
+import oracle
+from conftest import assert_close_absmax, from_dev_bf16, randn_bf16, to_dev_bf16
 from h3attn import ops, sla
 
 pytestmark = pytest.mark.gpu
@@ -83,3 +86,44 @@ def test_pooled_prologue_tokens_heads_edges(gpu, S, H, blk, rot):
     assert torch.equal(got, want)
     for m, x in zip(means, heads(want)):
         assert torch.equal(m, ops.block_pool(x.transpose(1, 2), blk))
+
+
+@pytest.mark.parametrize("B,H,Sq,Skv", [(1, 1, 1, 1), (1, 2, 63, 64), (1, 3, 65, 65), (2, 2, 64, 128), (1, 2, 300, 300),
+                                        (2, 3, 129, 191), (1, 28, 700, 700), (1, 1, 40, 3000), (1, 2, 1000, 1090),
+                                        (2, 14, 580, 1100)])
+def test_short_tiles_match_oracle(gpu, B, H, Sq, Skv):
+    """Launches of few tiles (128- and 64-row tiles, whole or in key ranges) at ragged rows and keys, down
+    to ranges in which one group has no stage."""
+    rng = np.random.default_rng(Sq + Skv)
+    q, k, v = (randn_bf16(rng, (B, H, n, 128)) for n in (Sq, Skv, Skv))
+    dev = [to_dev_bf16(x, gpu) for x in (q, k, v)]
+    out = torch.full((B, Sq, H, 128), float("nan"), dtype=torch.bfloat16, device=gpu).transpose(1, 2)
+    ops.attn_fwd(*dev, out=out)
+    got = oracle.bf16_to_f32(from_dev_bf16(out)).reshape(out.shape)
+    assert_close_absmax(got, oracle.attn_fwd(q, k, v), what=f"{B}x{H}x{Sq}x{Skv}")
+
+
+@pytest.mark.parametrize("H,Sq,Skv", [(1, 5000, 5000), (4, 8000, 4100), (10, 1500, 1500), (28, 2500, 2600), (3, 100, 20000)])
+def test_short_tiles_and_key_ranges_match_whole_tiles(gpu, H, Sq, Skv):
+    torch.manual_seed(H)
+    q, k, v = (torch.randn(1, H, n, 128, device=gpu).bfloat16() for n in (Sq, Skv, Skv))
+    got = ops.attn_fwd(q, k, v).float()
+    want = ops.attn_fwd(q, k, v, split_tail=False).float()
+    d = (got - want).abs()
+    # Both round O (2^-9 relative) and every p (2^-9 each, averaging out over the keys): on the mean
+    # the two differ by less than the sum of the four bounds.
+    assert d.max() <= 1e-2 * want.abs().max() and d.mean() <= 2.0 ** -7 * want.abs().mean()
+
+
+@pytest.mark.parametrize("H,Sq", [(1, 64), (3, 4000)])
+def test_short_tiles_wide_kv_stride(gpu, H, Sq):
+    """K/V whose rows lie so far apart that a slice passes 2^32 bytes (per-stage descriptors)."""
+    torch.manual_seed(1)
+    Skv, stride = 200, (1 << 23) + 8
+    buf = torch.empty(Skv * stride, dtype=torch.bfloat16, device=gpu)
+    q = torch.randn(1, H, Sq, 128, device=gpu).bfloat16()
+    k, v = (torch.randn(1, H, Skv, 128, device=gpu).bfloat16() for _ in range(2))
+    kw, vw = (buf.as_strided((1, H, Skv, 128), (0, 128, stride, 1), off * 128 * H) for off in (0, 1))
+    kw.copy_(k)
+    vw.copy_(v)
+    assert torch.equal(ops.attn_fwd(q, kw, vw), ops.attn_fwd(q, k, v))
