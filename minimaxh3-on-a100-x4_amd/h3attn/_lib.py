@@ -9,6 +9,7 @@ only maps it.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import threading
 
@@ -121,7 +122,9 @@ def check(fn: str, rc: int, handle: ctypes.CDLL | None = None) -> None:
         raise H3AError(fn, rc, msg)
 
 
+@functools.lru_cache(maxsize=1024)
 def strides3(a, b, c) -> ctypes.Array:
+    """int64[3] argument; shared between calls with the same values, so not to be written."""
     return _c_i64_3(int(a), int(b), int(c))
 
 

@@ -8,6 +8,7 @@ CPU fallback.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import math
 
@@ -19,61 +20,87 @@ from ._lib import check, lib, strides3
 HEAD_DIM = 128
 
 
-def _stream(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+# A call's own host work bounds the smallest problems (H=2, S=300: a kernel of
+# 9 us under 20 us of Python), so the checks below read shape and strides once per
+# tensor, the device is only switched where it differs, and the raw stream handle
+# is taken without a Stream object.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_SAME_DEVICE = contextlib.nullcontext()
 
 
-def _norm_stride(t: torch.Tensor, dim: int) -> int:
-    # A size-1 dimension is never stepped along; its stride is irrelevant.
-    return 0 if t.shape[dim] == 1 else t.stride(dim)
+def _stream(t: torch.Tensor) -> int:
+    if _raw_stream is not None:
+        return _raw_stream(t.get_device())
+    return torch.cuda.current_stream(t.device).cuda_stream
 
 
-def _kernel_ready(t: torch.Tensor, outer_dims) -> bool:
-    """Last dim unit-stride, base 16-byte aligned, outer strides multiples of 8."""
-    if t.stride(-1) != 1 or t.data_ptr() % 16 != 0:
-        return False
-    return all(_norm_stride(t, d) % 8 == 0 and _norm_stride(t, d) >= 0 for d in outer_dims)
+def _on_device(t: torch.Tensor):
+    """Context in which t's device is the current one."""
+    return _SAME_DEVICE if t.get_device() == torch.cuda.current_device() else torch.cuda.device(t.device)
 
 
-def _as_kernel_input(name: str, t: torch.Tensor) -> torch.Tensor:
+def _layout(t: torch.Tensor):
+    """Outer strides of a 4-D tensor the kernels can read or write in place, else None.
+
+    In place: last dim unit-stride, base 16-byte aligned, outer strides multiples of 8.
+    A size-1 dimension is never stepped along; its stride is irrelevant (0).
+    """
+    n0, n1, n2, _ = t.shape
+    s0, s1, s2, s3 = t.stride()
+    if n0 == 1:
+        s0 = 0
+    if n1 == 1:
+        s1 = 0
+    if n2 == 1:
+        s2 = 0
+    if s3 != 1 or (s0 | s1 | s2) & 7 or t.data_ptr() & 15:
+        return None
+    return s0, s1, s2
+
+
+def _as_kernel_input(name: str, t: torch.Tensor):
+    """t, or a contiguous copy where its layout cannot be streamed directly (same HIP path), and its strides."""
     if not isinstance(t, torch.Tensor):
         raise ValueError(f"{name} must be a torch.Tensor")
     if t.dim() != 4:
         raise ValueError(f"{name} must be 4-D [B,H,S,D], got shape {tuple(t.shape)}")
-    if t.shape[-1] != HEAD_DIM:
+    if t.shape[3] != HEAD_DIM:
         raise ValueError(f"{name}: head_dim {t.shape[-1]} unsupported (only {HEAD_DIM})")
     if t.dtype != torch.bfloat16:
         raise ValueError(f"{name} must be bfloat16, got {t.dtype}")
     if not t.is_cuda:
         raise ValueError(f"{name} must be a GPU tensor (libh3attn has no CPU path)")
-    # Layouts the kernel cannot stream directly are made contiguous (same HIP path).
-    return t if _kernel_ready(t, (0, 1, 2)) else t.contiguous()
-
-
-def _bhs(t: torch.Tensor):
-    return strides3(_norm_stride(t, 0), _norm_stride(t, 1), _norm_stride(t, 2))
+    st = _layout(t)
+    if st is None:
+        t = t.contiguous()
+        st = t.stride()[:3]  # (a base off the 16-byte grid is refused by the entry point)
+    return t, strides3(*st)
 
 
 def _prepare_attn(q, k, v, out):
-    q = _as_kernel_input("q", q)
-    k = _as_kernel_input("k", k)
-    v = _as_kernel_input("v", v)
-    B, H, Sq, D = q.shape
-    Skv = k.shape[2]
-    if tuple(k.shape) != (B, H, Skv, D) or tuple(v.shape) != (B, H, Skv, D):
+    q, qst = _as_kernel_input("q", q)
+    k, kst = _as_kernel_input("k", k)
+    v, vst = _as_kernel_input("v", v)
+    B, H, Sq, D = shape = q.shape
+    kshape = k.shape
+    Skv = kshape[2]
+    if kshape != v.shape or kshape[0] != B or kshape[1] != H:
         raise ValueError(f"shape mismatch: q {tuple(q.shape)} k {tuple(k.shape)} v {tuple(v.shape)}")
     if Sq == 0 or Skv == 0 or B == 0 or H == 0:
         raise ValueError("empty attention input")
-    if not (q.device == k.device == v.device):
+    device = q.device
+    if not (device == k.device == v.device):
         raise ValueError("q, k, v must be on the same device")
     if out is None:
-        out = torch.empty((B, H, Sq, D), dtype=torch.bfloat16, device=q.device)
+        out = torch.empty(shape, dtype=torch.bfloat16, device=device)
+        ost = (0 if B == 1 else H * Sq * D, 0 if H == 1 else Sq * D, 0 if Sq == 1 else D)
     else:
-        if tuple(out.shape) != (B, H, Sq, D) or out.dtype != torch.bfloat16 or out.device != q.device:
+        if out.shape != shape or out.dtype != torch.bfloat16 or out.device != device:
             raise ValueError("out must be a bf16 [B,H,Sq,128] tensor on q's device")
-        if not _kernel_ready(out, (0, 1, 2)):
+        ost = _layout(out)
+        if ost is None:
             raise ValueError("out must have unit last stride, 16-byte alignment and strides multiple of 8")
-    return q, k, v, out, (B, H, Sq, Skv, D)
+    return q, k, v, out, (B, H, Sq, Skv, D), (qst, kst, vst, strides3(*ost))
 
 
 def attn_workspace_bytes(B: int, H: int, Sq: int, Skv: int, D: int = HEAD_DIM) -> int:
@@ -96,11 +123,11 @@ def attn_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: float | N
     split along the keys (equal results up to rounding); False runs
     h3a_attn_fwd, which never splits.
     """
-    q, k, v, out, (B, H, Sq, Skv, D) = _prepare_attn(q, k, v, out)
+    q, k, v, out, (B, H, Sq, Skv, D), st = _prepare_attn(q, k, v, out)
     sc = 1.0 / math.sqrt(D) if scale is None else float(scale)
     args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-            B, H, Sq, Skv, D, _bhs(q), _bhs(k), _bhs(v), _bhs(out), sc)
-    with torch.cuda.device(q.device):
+            B, H, Sq, Skv, D, *st, sc)
+    with _on_device(q):
         if split_tail:
             nbytes = attn_workspace_bytes(B, H, Sq, Skv, D)
             ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
@@ -124,12 +151,12 @@ def attn_fwd_profiled(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scale: 
     prof_read().  The profile build stamps the shader clock inside the stage
     loop, so it runs a little slower than the product build.
     """
-    q, k, v, out, (B, H, Sq, Skv, D) = _prepare_attn(q, k, v, out)
+    q, k, v, out, (B, H, Sq, Skv, D), st = _prepare_attn(q, k, v, out)
     sc = 1.0 / math.sqrt(D) if scale is None else float(scale)
     L = lib(profile=True)
-    with torch.cuda.device(q.device):
+    with _on_device(q):
         rc = L.h3a_attn_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, H, Sq, Skv, D,
-                            _bhs(q), _bhs(k), _bhs(v), _bhs(out), sc, _stream(q))
+                            *st, sc, _stream(q))
     check("h3a_attn_fwd (profile build)", rc, L)
     return out
 
@@ -141,13 +168,13 @@ def attn_fwd_blocksparse_profiled(q, k, v, lut, counts, blk_q: int, blk_k: int, 
     The ping-pong sparse kernels (pairs of query blocks) record workgroup 0's
     per-wave phases like the dense kernel; read them with prof_read().
     """
-    q, k, v, out, (B, H, Sq, Skv, D) = _prepare_attn(q, k, v, out)
+    q, k, v, out, (B, H, Sq, Skv, D), st = _prepare_attn(q, k, v, out)
     lut, counts = lut.contiguous(), counts.contiguous()
     sc = 1.0 / math.sqrt(D) if scale is None else float(scale)
     L = lib(profile=True)
-    with torch.cuda.device(q.device):
+    with _on_device(q):
         rc = L.h3a_attn_fwd_blocksparse(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, H, Sq, Skv,
-                                        D, _bhs(q), _bhs(k), _bhs(v), _bhs(out), lut.data_ptr(), counts.data_ptr(),
+                                        D, *st, lut.data_ptr(), counts.data_ptr(),
                                         int(blk_q), int(blk_k), int(lut.shape[3]), sc, _stream(q))
     check("h3a_attn_fwd_blocksparse (profile build)", rc, L)
     return out
@@ -156,13 +183,13 @@ def attn_fwd_blocksparse_profiled(q, k, v, lut, counts, blk_q: int, blk_k: int, 
 def attn_fwd_blocksparse_tiles_profiled(q, k, v, tile_lut, tile_counts, scale: float | None = None,
                                         out: torch.Tensor | None = None) -> torch.Tensor:
     """attn_fwd_blocksparse_tiles through the phase-profile build (h3a_attn_fwd_blocksparse_tiles)."""
-    q, k, v, out, (B, H, Sq, Skv, D) = _prepare_attn(q, k, v, out)
+    q, k, v, out, (B, H, Sq, Skv, D), st = _prepare_attn(q, k, v, out)
     tile_lut, tile_counts = tile_lut.contiguous(), tile_counts.contiguous()
     sc = 1.0 / math.sqrt(D) if scale is None else float(scale)
     L = lib(profile=True)
-    with torch.cuda.device(q.device):
+    with _on_device(q):
         rc = L.h3a_attn_fwd_blocksparse_tiles(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, H, Sq,
-                                              Skv, D, _bhs(q), _bhs(k), _bhs(v), _bhs(out), tile_lut.data_ptr(),
+                                              Skv, D, *st, tile_lut.data_ptr(),
                                               tile_counts.data_ptr(), int(tile_lut.shape[3]), sc, _stream(q))
     check("h3a_attn_fwd_blocksparse_tiles (profile build)", rc, L)
     return out
@@ -229,7 +256,7 @@ def attn_fwd_blocksparse(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, lut:
         bmap = lut_to_block_map(lut, counts, -(-Skv // blk_k))
         tlut, tcnt = block_map_to_tile_lut(bmap, blk_q, blk_k, Sq, Skv)
         return attn_fwd_blocksparse_tiles(q, k, v, tlut, tcnt, scale=scale, out=out, queues=split_tail)
-    q, k, v, out, (B, H, Sq, Skv, D) = _prepare_attn(q, k, v, out)
+    q, k, v, out, (B, H, Sq, Skv, D), st = _prepare_attn(q, k, v, out)
     nqb = -(-Sq // blk_q)
     if lut.dtype != torch.int32 or counts.dtype != torch.int32:
         raise ValueError("lut and counts must be int32")
@@ -243,9 +270,9 @@ def attn_fwd_blocksparse(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, lut:
     counts = counts.contiguous()
     sc = 1.0 / math.sqrt(D) if scale is None else float(scale)
     args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, H, Sq, Skv, D,
-            _bhs(q), _bhs(k), _bhs(v), _bhs(out), lut.data_ptr(), counts.data_ptr(),
+            *st, lut.data_ptr(), counts.data_ptr(),
             int(blk_q), int(blk_k), int(lut.shape[3]), sc)
-    with torch.cuda.device(q.device):
+    with _on_device(q):
         nbytes = (sparse_workspace_bytes(B, H, Sq, Skv, blk_q, blk_k, int(lut.shape[3]), D)
                   if split_tail else 0)
         if nbytes:
@@ -280,7 +307,7 @@ def attn_fwd_blocksparse_tiles(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
     h3a_attn_fwd_blocksparse_tiles (sub-blocks 2p and 2p+1 paired).  Both give
     the same output bit for bit.
     """
-    q, k, v, out, (B, H, Sq, Skv, D) = _prepare_attn(q, k, v, out)
+    q, k, v, out, (B, H, Sq, Skv, D), st = _prepare_attn(q, k, v, out)
     nsub = -(-Sq // 64)
     if tile_lut.dtype != torch.int32 or tile_counts.dtype != torch.int32:
         raise ValueError("tile_lut and tile_counts must be int32")
@@ -294,8 +321,8 @@ def attn_fwd_blocksparse_tiles(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
     sc = 1.0 / math.sqrt(D) if scale is None else float(scale)
     max_tiles = int(tile_lut.shape[3])
     args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, H, Sq, Skv, D,
-            _bhs(q), _bhs(k), _bhs(v), _bhs(out), tile_lut.data_ptr(), tile_counts.data_ptr(), max_tiles, sc)
-    with torch.cuda.device(q.device):
+            *st, tile_lut.data_ptr(), tile_counts.data_ptr(), max_tiles, sc)
+    with _on_device(q):
         nbytes = tiles_workspace_bytes(B, H, Sq, Skv, max_tiles, D) if queues else 0
         if nbytes:
             ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
@@ -368,10 +395,10 @@ def block_map_to_lut(block_map: torch.Tensor, max_k_blocks: int | None = None):
 
 def block_pool(x: torch.Tensor, blk: int) -> torch.Tensor:
     """Block means over the valid rows of each block: bf16 [B,H,S,128] -> fp32 [B,H,ceil(S/blk),128]."""
-    x = _as_kernel_input("x", x)
+    x, st = _as_kernel_input("x", x)
     B, H, S, D = x.shape
     out = torch.empty((B, H, -(-S // blk), D), dtype=torch.float32, device=x.device)
-    rc = lib().h3a_block_pool(x.data_ptr(), B, H, S, D, _bhs(x), int(blk), out.data_ptr(), _stream(x))
+    rc = lib().h3a_block_pool(x.data_ptr(), B, H, S, D, st, int(blk), out.data_ptr(), _stream(x))
     check("h3a_block_pool", rc)
     return out
 
@@ -443,12 +470,15 @@ def qk_rmsnorm_rope_(q: torch.Tensor, k: torch.Tensor, rope: torch.Tensor | None
     block means (q_means, k_means) [B,H,ceil(S/pool_blk),128], equal to
     block_pool of the updated q and k (as [B,H,S,128]).
     """
+    sts = []
     for name, t in (("q", q), ("k", k)):
         if t.dtype != torch.bfloat16 or not t.is_cuda or t.dim() != 4 or t.shape[-1] != HEAD_DIM:
             raise ValueError(f"{name} must be a bf16 GPU tensor [B,S,H,128], got {t.dtype} {tuple(t.shape)}")
-        if not _kernel_ready(t, (0, 1, 2)):
+        st = _layout(t)
+        if st is None:
             raise ValueError(f"{name}: in-place update needs unit last stride, 16-byte alignment and "
                              "outer strides that are multiples of 8 elements")
+        sts.append(strides3(*st))
     if tuple(q.shape) != tuple(k.shape):
         raise ValueError("q and k must have the same shape")
     B, S, H, D = q.shape
@@ -459,18 +489,18 @@ def qk_rmsnorm_rope_(q: torch.Tensor, k: torch.Tensor, rope: torch.Tensor | None
     for name, w in (("qw", qw), ("kw", kw)):
         if w.numel() != D:
             raise ValueError(f"{name} must have {D} elements")
-        w = w.reshape(D).to(device=q.device, dtype=torch.bfloat16).contiguous()
+        if w.dtype != torch.bfloat16 or w.device != q.device or not w.is_contiguous():
+            w = w.reshape(D).to(device=q.device, dtype=torch.bfloat16).contiguous()
         ws.append(w)
     if rot_dim > 0:
         if rope is None:
             raise ValueError("rope table required when rot_dim > 0")
-        rope, rsb, rss = _rope_table(rope.to(q.device), B, S, rot_dim)
+        rope, rsb, rss = _rope_table(rope if rope.device == q.device else rope.to(q.device), B, S, rot_dim)
         rptr = rope.data_ptr()
     else:
         rptr, rsb, rss = None, 0, 0
     args = (q.data_ptr(), k.data_ptr(), B, S, H, D,
-            strides3(_norm_stride(q, 0), _norm_stride(q, 1), _norm_stride(q, 2)),
-            strides3(_norm_stride(k, 0), _norm_stride(k, 1), _norm_stride(k, 2)),
+            *sts,
             rptr, int(rsb), int(rss), rot_dim, ws[0].data_ptr(), ws[1].data_ptr(), float(eps))
     if pool_blk is None:
         check("h3a_qk_rmsnorm_rope", lib().h3a_qk_rmsnorm_rope(*args, _stream(q)))
