@@ -1695,47 +1695,39 @@ __global__ void __launch_bounds__(256) block_map_row_max_kernel(const uint8_t *m
 // stages as the longer of its two lists, so a pair of unequal lists leaves
 // one group idle for the difference: with blk_q 80, 96, 112, 144, ... a block
 // boundary falls inside some sub-blocks and not others, and those hold the
-// union of two blocks' lists.  One workgroup per (b,h) sorts its sub-blocks
-// by stage count, descending (ties by index), in LDS (bitonic), and pairs
-// neighbours: map[bh][p] = sorted entries 2p and 2p+1, an odd count pairing
-// the last with sub-block nsub, which has no rows.  Which sub-blocks share a
+// union of two blocks' lists.  So the sub-blocks of every run of 64 (one wave's
+// lanes) are ranked by stage count, descending (ties by index), and neighbours
+// paired: map[bh][p] = ranked entries 2p and 2p+1, an odd count pairing the
+// last with sub-block nsub, which has no rows.  Which sub-blocks share a
 // workgroup does not change any row's arithmetic.
-__global__ void __launch_bounds__(1024) tile_pair_map_kernel(const int32_t *counts, int nsub, int lut_stride,
-                                                             int32_t *map) {
-  __shared__ uint32_t key[kPairSortMax];
-  const int tid = threadIdx.x;
-  const int64_t bh = blockIdx.x;
-  int n = 2;
-  while (n < nsub) n <<= 1;
-  const int32_t *c = counts + bh * nsub;
-  for (int i = tid; i < n; i += 1024) {
-    uint32_t kv = 0xffffffffu;  // padding sorts last
-    if (i < nsub) {
-      const int e = c[i] < 0 ? 0 : (c[i] > lut_stride ? lut_stride : c[i]);
-      const uint32_t st = (uint32_t)(e + 1) / 2;  // stages, <= 32767
-      kv = ((0x7fffu - st) << 16) | (uint32_t)i;
-    }
-    key[i] = kv;
+//
+// Runs of 64, not whole heads: the 32 CUs of an XCD take 32 consecutive pairs
+// and share its L2, and sub-blocks far apart in the sequence keep different key
+// blocks.  Against ranking all of a head's sub-blocks, at H=28 S=42120, keep
+// 0.25: 96x96 8.24 -> 8.11 ms, 80x80 9.41 -> 9.12, 112x112 9.18 -> 8.88, 48x48
+// 10.13 -> 10.06, 208x208 8.18 -> 8.23 (keep 0.15 at 32x32 5.98 -> 5.94).  Runs of
+// 32 measured 1-11 % slower than runs of 64, runs of 128 and 256 0-5 %.  The
+// ranking itself, one wave per run instead of a sort in LDS per head, takes
+// 4 us instead of 18.
+constexpr int kPairRun = 64;
+__global__ void __launch_bounds__(256) tile_pair_map_kernel(const int32_t *counts, int64_t runs, int runs_bh, int nsub,
+                                                            int lut_stride, int32_t *map) {
+  const int lane = threadIdx.x & 63;
+  const int64_t run = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (run >= runs) return;  // whole waves leave together
+  const int64_t bh = run / runs_bh;
+  const int i0 = (int)(run % runs_bh) * kPairRun, i = i0 + lane;
+  uint32_t key = 0xffffffc0u | (uint32_t)lane;  // past the end: last
+  if (i < nsub) {
+    const int c = counts[bh * nsub + i];
+    const int e = c < 0 ? 0 : (c > lut_stride ? lut_stride : c);
+    key = (0xffffu - (uint32_t)((e + 1) / 2)) << 6 | (uint32_t)lane;  // stages <= 32767
   }
-  __syncthreads();
-  for (int k = 2; k <= n; k <<= 1) {
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int i = tid; i < n; i += 1024) {
-        const int l = i ^ j;
-        if (l > i) {
-          const uint32_t x = key[i], y = key[l];
-          if ((i & k) == 0 ? x > y : x < y) {
-            key[i] = y;
-            key[l] = x;
-          }
-        }
-      }
-      __syncthreads();
-    }
-  }
-  const int npairs = (nsub + 1) / 2;
-  int32_t *out = map + bh * npairs * 2;
-  for (int t = tid; t < 2 * npairs; t += 1024) out[t] = t < nsub ? (int32_t)(key[t] & 0xffffu) : nsub;
+  int rank = 0;
+#pragma unroll
+  for (int j = 0; j < kPairRun; ++j) rank += (uint32_t)__builtin_amdgcn_readlane((int)key, j) < key;
+  const int entries = 2 * ((nsub + 1) / 2);
+  if (i0 + rank < entries) map[bh * entries + i0 + rank] = i < nsub ? i : nsub;
 }
 
 // ---------------------------------------------------------------------------
@@ -2003,8 +1995,10 @@ int launch_attn_sparse_split(const AttnArgs &a, int blk_q, const SplitPlan &plan
   AttnArgs p = a;
   if (tiles && plan.pair_map) {
     int32_t *map = static_cast<int32_t *>(ws);
-    hipLaunchKernelGGL(tile_pair_map_kernel, dim3((unsigned)(a.B * a.H)), dim3(1024), 0, s, a.counts, a.nqt,
-                       a.lut_stride, map);
+    const int runs_bh = (a.nqt + kPairRun - 1) / kPairRun;
+    const int64_t runs = (int64_t)a.B * a.H * runs_bh;
+    hipLaunchKernelGGL(tile_pair_map_kernel, dim3((unsigned)((runs + 3) / 4)), dim3(256), 0, s, a.counts, runs,
+                       runs_bh, a.nqt, a.lut_stride, map);
     const int rc = check_launch("tile_pair_map_kernel");
     if (rc) return rc;
     p.pair_map = map;

@@ -66,8 +66,8 @@ inline bool tile_block_ok(int blk) { return blk > 0 && blk % 16 == 0; }
 // 32-key columns a tile LUT entry can name (column << 8 | mask stays positive
 // and below 2^24): Skv <= kMaxTileColumns * 32.
 constexpr int kMaxTileColumns = 65534;
-// Query sub-blocks per (b,h) whose pairing by stage count is sorted in one
-// workgroup's LDS (tile path; longer sequences pair sub-blocks 2p, 2p+1).
+// Query sub-blocks per (b,h) up to which they are paired by stage count (tile
+// path; longer sequences pair sub-blocks 2p, 2p+1).
 constexpr int kPairSortMax = 16384;
 inline int sparse_sub_block_rows(int blk_q) { return blk_q % 128 == 0 ? 128 : 64; }
 
