@@ -1187,7 +1187,11 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
   auto soft = [&](int j) __attribute__((always_inline)) {
     // Tile masks: the keys are already this wave's own column's.
     const int key0 = (kSparse ? soft_key : key_base(j + 1)) + (kTileMask ? 0 : 32 * kh);
-    if constexpr (kTileMask) apply_tile_mask<WS>(s, soft_mask, rq, l32);
+    // Most columns are kept whole for the wave's 32 rows (the mask's four bits):
+    // skipping their 16 selects shortens the stage's softmax: at H=28 S=42120, keep 0.25, 96x96
+    // 8.42 -> 8.07 ms, 80x80 9.43 -> 9.18, 48x48 10.40 -> 10.15, 144x144 8.90 -> 8.63.
+    if constexpr (kTileMask)
+      if (((soft_mask >> (4 * rq)) & 0xfu) != 0xfu) apply_tile_mask<WS>(s, soft_mask, rq, l32);
     softmax_stage_stale<WS, kSparse>(s, key0, a.Skv, g, a.sl2, m, lsum, o, pf);
 #pragma unroll
     for (int i = 0; i < 2 * WS; ++i) pin(pf[i]);
