@@ -220,8 +220,8 @@ __global__ void __launch_bounds__(NW * 64, NW == kSelMidWaves ? 4 : 1) block_sel
   // Rows of up to NC*64 key blocks: the keys of all of this wave's rows
   // (wave + NW*i, i < RPW) sit in registers, NC per lane per row, and the
   // rows' searches run interleaved, so their 32 dependent counting rounds
-  // overlap.  (NC, RPW) = (6, 4) or (12, 4) with 4 waves, (24, 2) with 8,
-  // (48, 1) with 16: at most 48 registers of keys, for 16 rows.
+  // overlap.  NC = 2, 6 or 12 and RPW = 1, 2 or 4 with 4 waves, (24, 2) with
+  // 8, (48, 1) with 16: at most 48 registers of keys, for 16 rows.
   auto select_rows_regs = [&](auto nc_const, auto rpw_const) __attribute__((always_inline)) {
     constexpr int NC = decltype(nc_const)::value;
     constexpr int RPW = decltype(rpw_const)::value;
@@ -318,10 +318,20 @@ __global__ void __launch_bounds__(NW * 64, NW == kSelMidWaves ? 4 : 1) block_sel
     else
       select_rows_lds();
   } else {
-    if (nchunks <= 6)
-      select_rows_regs(std::integral_constant<int, 6>{}, I4{});
+    auto select_rows = [&](auto nc_const) __attribute__((always_inline)) {
+      if (R <= NW)
+        select_rows_regs(nc_const, I1{});
+      else if (R <= 2 * NW)
+        select_rows_regs(nc_const, I2{});
+      else
+        select_rows_regs(nc_const, I4{});
+    };
+    if (nchunks <= 2)
+      select_rows(I2{});
+    else if (nchunks <= 6)
+      select_rows(std::integral_constant<int, 6>{});
     else if (nchunks <= 12)
-      select_rows_regs(std::integral_constant<int, 12>{}, I4{});
+      select_rows(std::integral_constant<int, 12>{});
     else
       select_rows_lds();
   }
@@ -501,6 +511,21 @@ int launch_block_select(const float *pq, const float *pk, int B, int H, int nq, 
   }
   int rows = kSelScoreBytes / (nk * (int)sizeof(float));
   rows = rows < 1 ? 1 : (rows > kSelRowsMax ? kSelRowsMax : rows);
+  // Fewer rows per workgroup while the whole launch is still resident: a wave
+  // selects its rows one after another, which is most of a short launch (the
+  // search's 32 dependent counting rounds, the row's output), and the pooled keys
+  // that every workgroup reads are few.  16 / 8 / 4 rows: 15.3 / 9.3 / 5.9 us at 14
+  // heads of 65 blocks (70 to 238 workgroups), 18.2 / 13.5 / 8.4 at 4 of 157, but
+  // 33.3 / 32.4 / 36.9 at 14 of 330 (294 / 588 / 1162) and 67 / 74 / 108 at 14 of
+  // 659 (616 / 1162 / 2310); past 640 key blocks the scores take most of the time
+  // (4 heads of 760: 42.0 / 43.6 / 44.7).
+  constexpr int64_t kSelResident = 1024;  // four workgroups per CU
+  for (int r = kSelThreads / 64; nk <= 640 && r <= 2 * (kSelThreads / 64); r *= 2) {
+    if (r < rows && (int64_t)B * H * ((nq + r - 1) / r) <= kSelResident) {
+      rows = r;
+      break;
+    }
+  }
   const size_t lds = ((size_t)rows * nk + 1) * sizeof(float);
   const int64_t groups = (int64_t)B * H * ((nq + rows - 1) / rows);
   hipLaunchKernelGGL(block_select_kernel<kSelThreads / 64>, dim3((unsigned)groups), dim3(kSelThreads), lds, s,

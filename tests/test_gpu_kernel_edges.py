@@ -127,3 +127,23 @@ def test_short_tiles_wide_kv_stride(gpu, H, Sq):
     kw.copy_(k)
     vw.copy_(v)
     assert torch.equal(ops.attn_fwd(q, kw, vw), ops.attn_fwd(q, k, v))
+
+
+@pytest.mark.parametrize("H,nq,nk", [(1, 1, 1), (2, 5, 64), (3, 17, 128), (14, 65, 65), (4, 33, 129), (60, 65, 65),
+                                     (140, 65, 40), (30, 157, 385), (5, 40, 768)])
+def test_block_select_rows_per_workgroup(gpu, H, nq, nk):
+    """Block selection in workgroups of 4, 8 and 16 rows (by how many there are), on integer vectors, where
+    every order of summation gives the same scores and ties abound."""
+    g = torch.Generator().manual_seed(nk)
+    pq, pk = (torch.randint(-2, 3, (1, H, n, 128), generator=g).float() for n in (nq, nk))
+    keep = max(1, nk // 3)
+    bmap, lut, cnt = ops.block_select(pq.to(gpu), pk.to(gpu), keep, 64, 64, force_diag=True)
+    score = pq @ pk.transpose(2, 3)
+    want = torch.zeros(1, H, nq, nk, dtype=torch.uint8)
+    want.scatter_(3, score.sort(dim=3, descending=True, stable=True).indices[..., :keep], 1)
+    d = torch.arange(min(nq, nk))
+    want[:, :, d, d] = 1
+    assert torch.equal(bmap.cpu(), want)
+    assert torch.equal(cnt.cpu(), want.sum(3, dtype=torch.int32))
+    idx = torch.where(want.bool(), torch.arange(nk), nk).sort(3).values[..., :lut.shape[3]]
+    assert torch.equal(lut.cpu(), torch.where(idx < nk, idx, -1).int())
