@@ -196,7 +196,7 @@ int h3a_attn_fwd_blocksparse_ws(const void *q, const void *k, const void *v, voi
  * The kernel runs two rows (64-row sub-blocks) per workgroup for as many
  * stages as the longer of the two; h3a_attn_fwd_blocksparse_tiles pairs rows
  * 2p and 2p+1, the _ws variant pairs them by length (a kernel ranks each
- * run of 64 rows into the workspace first; up to ceil(Sq/64) = 16384, beyond
+ * run of 128 rows into the workspace first; up to ceil(Sq/64) = 16384, beyond
  * that as the plain call).  Results are the same bit for bit; the workspace
  * is never 0 bytes then.
  * No counterpart in the reference's own code: SLA's Triton kernel takes the

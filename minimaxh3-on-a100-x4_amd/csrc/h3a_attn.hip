@@ -1699,39 +1699,56 @@ __global__ void __launch_bounds__(256) block_map_row_max_kernel(const uint8_t *m
 // stages as the longer of its two lists, so a pair of unequal lists leaves
 // one group idle for the difference: with blk_q 80, 96, 112, 144, ... a block
 // boundary falls inside some sub-blocks and not others, and those hold the
-// union of two blocks' lists.  So the sub-blocks of every run of 64 (one wave's
-// lanes) are ranked by stage count, descending (ties by index), and neighbours
-// paired: map[bh][p] = ranked entries 2p and 2p+1, an odd count pairing the
-// last with sub-block nsub, which has no rows.  Which sub-blocks share a
-// workgroup does not change any row's arithmetic.
+// union of two blocks' lists.  So the sub-blocks of every run of 128 (two per
+// lane of a wave) are ranked by stage count, descending (ties by index), and
+// neighbours paired: map[bh][p] = ranked entries 2p and 2p+1, an odd count
+// pairing the last with sub-block nsub, which has no rows.  Which sub-blocks
+// share a workgroup does not change any row's arithmetic.
 //
-// Runs of 64, not whole heads: the 32 CUs of an XCD take 32 consecutive pairs
-// and share its L2, and sub-blocks far apart in the sequence keep different key
-// blocks.  Against ranking all of a head's sub-blocks, at H=28 S=42120, keep
-// 0.25: 96x96 8.24 -> 8.11 ms, 80x80 9.41 -> 9.12, 112x112 9.18 -> 8.88, 48x48
-// 10.13 -> 10.06, 208x208 8.18 -> 8.23 (keep 0.15 at 32x32 5.98 -> 5.94).  Runs of
-// 32 measured 1-11 % slower than runs of 64, runs of 128 and 256 0-5 %.  The
-// ranking itself, one wave per run instead of a sort in LDS per head, takes
-// 4 us instead of 18.
-constexpr int kPairRun = 64;
+// Runs, not whole heads: the 32 CUs of an XCD take 32 consecutive pairs and
+// share its L2, and sub-blocks far apart in the sequence keep different key
+// blocks.  Short runs balance the pairs less, the more so the less neighbouring
+// lists agree.  Runs of 64 / 128 / 256 / a whole head at H=28 S=42120, keep 0.25:
+// on a layer's q and k 96x96 7.65 / 7.63 / 7.83 / 7.81 ms, 80x80 8.71 / 8.97 / 9.01 /
+// 9.66, 144x144 8.21 / 8.17 / 8.24 / 8.25, 48x48 9.63 / 9.80 / 9.87 / 9.79; on lists
+// that hardly agree 96x96 8.63 / 8.34 / 8.37 / 8.17, 144x144 9.13 / 8.96 / 8.85 /
+// 8.84.  The ranking itself takes 4 us, a sort in LDS per head took 18.
+constexpr int kPairPer = 2;  // sub-blocks per lane
+constexpr int kPairRun = 64 * kPairPer;
 __global__ void __launch_bounds__(256) tile_pair_map_kernel(const int32_t *counts, int64_t runs, int runs_bh, int nsub,
                                                             int lut_stride, int32_t *map) {
   const int lane = threadIdx.x & 63;
   const int64_t run = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (run >= runs) return;  // whole waves leave together
   const int64_t bh = run / runs_bh;
-  const int i0 = (int)(run % runs_bh) * kPairRun, i = i0 + lane;
-  uint32_t key = 0xffffffc0u | (uint32_t)lane;  // past the end: last
-  if (i < nsub) {
-    const int c = counts[bh * nsub + i];
-    const int e = c < 0 ? 0 : (c > lut_stride ? lut_stride : c);
-    key = (0xffffu - (uint32_t)((e + 1) / 2)) << 6 | (uint32_t)lane;  // stages <= 32767
-  }
-  int rank = 0;
+  const int i0 = (int)(run % runs_bh) * kPairRun;
+  uint32_t key[kPairPer];
+  int rank[kPairPer];
 #pragma unroll
-  for (int j = 0; j < kPairRun; ++j) rank += (uint32_t)__builtin_amdgcn_readlane((int)key, j) < key;
+  for (int u = 0; u < kPairPer; ++u) {
+    const int l = 64 * u + lane, i = i0 + l;
+    key[u] = 0xffff0000u | (uint32_t)l;  // past the end: last
+    rank[u] = 0;
+    if (i < nsub) {
+      const int c = counts[bh * nsub + i];
+      const int e = c < 0 ? 0 : (c > lut_stride ? lut_stride : c);
+      key[u] = (0x7fffu - (uint32_t)((e + 1) / 2)) << 16 | (uint32_t)l;  // stages <= 32767
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < kPairPer; ++v)
+#pragma unroll
+    for (int j = 0; j < 64; ++j) {
+      const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)key[v], j);
+#pragma unroll
+      for (int u = 0; u < kPairPer; ++u) rank[u] += other < key[u];
+    }
   const int entries = 2 * ((nsub + 1) / 2);
-  if (i0 + rank < entries) map[bh * entries + i0 + rank] = i < nsub ? i : nsub;
+#pragma unroll
+  for (int u = 0; u < kPairPer; ++u) {
+    const int i = i0 + 64 * u + lane;
+    if (i0 + rank[u] < entries) map[bh * entries + i0 + rank[u]] = i < nsub ? i : nsub;
+  }
 }
 
 // ---------------------------------------------------------------------------
