@@ -69,8 +69,16 @@ __host__ __device__ constexpr int rope_heads_per_wave(int H) { return H % 28 == 
 // The lane's half of its token's 2x2 matrices: lanes of the first rotated half
 // (c < nh) apply the first row (R00, R01), their partners the second (R10, R11).
 // Lanes past the rotated dims hold nothing.
+// kRot128: every dim is rotated (nh = 8), so neither this nor the row needs a
+// branch: branches between a token's loads and its use make the compiler wait
+// for more loads than the token's own.
+template <bool kRot128>
 __device__ __forceinline__ void load_rope(float2 (&R)[8], const float *rope_row, int c, int nh) {
-  if (c < 2 * nh) {
+  if (kRot128) {
+    const float *p = rope_row + (c & 7) * 32 + (c >> 3) * 2;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) R[e] = *(const float2 *)(p + 4 * e);
+  } else if (c < 2 * nh) {
     const float *p = rope_row + (c < nh ? c * 32 : (c - nh) * 32 + 2);
 #pragma unroll
     for (int e = 0; e < 8; ++e) R[e] = *(const float2 *)(p + 4 * e);
@@ -81,6 +89,7 @@ __device__ __forceinline__ void load_rope(float2 (&R)[8], const float *rope_row,
 }
 
 // y = rmsnorm(x) * w, then rotate pairs (i, i+rot/2) with the lane's matrix rows.
+template <bool kRot128>
 __device__ __forceinline__ void norm_rope_row(float (&x)[8], const float (&w)[8], float eps,
                                               const float2 (&R)[8], int c, int nh) {
   float ss = 0.f;
@@ -94,7 +103,7 @@ __device__ __forceinline__ void norm_rope_row(float (&x)[8], const float (&w)[8]
   const bool first = c < nh;
   const bool rotated = c < 2 * nh;
   float xp[8];
-  if (nh == 8) {  // rot = 128: the partner is 8 lanes away
+  if (kRot128) {  // the partner is 8 lanes away
 #pragma unroll
     for (int e = 0; e < 8; ++e) xp[e] = dpp_row<kDppRor8>(x[e]);
   } else {
@@ -102,13 +111,13 @@ __device__ __forceinline__ void norm_rope_row(float (&x)[8], const float (&w)[8]
 #pragma unroll
     for (int e = 0; e < 8; ++e) xp[e] = __shfl(x[e], partner, 16);
   }
-  if (rotated) {
+  if (kRot128 || rotated) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) x[e] = fmaf(R[e].x, first ? x[e] : xp[e], R[e].y * (first ? xp[e] : x[e]));
   }
 }
 
-template <int kHeadsPerWave>
+template <int kHeadsPerWave, bool kRot128>
 __global__ void __launch_bounds__(256) qk_rmsnorm_rope_kernel(RopeArgs a) {
   static_assert(kHeadsPerWave % 4 == 0, "four 16-lane groups per wave");
   constexpr int kSteps = kHeadsPerWave / 4;  // heads per 16-lane group
@@ -125,7 +134,7 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_kernel(RopeArgs a) {
   unpack8(*(const u32x4 *)(a.kw + c * 8), wk);
   float2 R[8];
   const int nh = a.rot >> 4;
-  load_rope(R, a.rope + b * a.rsb + s * a.rss, c, nh);
+  load_rope<kRot128>(R, a.rope + b * a.rsb + s * a.rss, c, nh);
 
   uint16_t *qrow = a.q + b * a.qsb + s * a.qss + c * 8;
   uint16_t *krow = a.k + b * a.ksb + s * a.kss + c * 8;
@@ -144,8 +153,8 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_kernel(RopeArgs a) {
     float xq[8], xk[8];
     unpack8(qv[i], xq);
     unpack8(kv[i], xk);
-    norm_rope_row(xq, wq, a.eps, R, c, nh);
-    norm_rope_row(xk, wk, a.eps, R, c, nh);
+    norm_rope_row<kRot128>(xq, wq, a.eps, R, c, nh);
+    norm_rope_row<kRot128>(xk, wk, a.eps, R, c, nh);
     if (heads[i] < a.H) {
       *(u32x4 *)(qrow + heads[i] * a.qsh) = pack8(xq);
       *(u32x4 *)(krow + heads[i] * a.ksh) = pack8(xk);
@@ -166,10 +175,10 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_kernel(RopeArgs a) {
 // tokens at small ones, so the loads of the next kDepth tokens are in flight
 // while one is computed (they come before its stores, which the compiler cannot
 // reorder) and the cross-lane steps stay in the VALU.  Per call, against loads,
-// LDS shuffles and stores token by token: H=14 S=4104 45.1 -> 27.8 us, H=56 S=4104
-// 67.2 -> 55.8, H=28 S=42120 (blocks of 96) 299 -> 269, H=56 S=42120 510 -> 502
+// LDS shuffles and stores token by token: H=14 S=4104 45.1 -> 24.7 us, H=56 S=4104
+// 67.2 -> 55.8, H=28 S=42120 (blocks of 96) 299 -> 266, H=56 S=42120 510 -> 501
 // (4.9 TB/s; a 2 GiB copy moves 5.0 on the same card).
-template <int kHeadsPerWave, int kDepth>
+template <int kHeadsPerWave, int kDepth, bool kRot128>
 __global__ void __launch_bounds__(256) qk_rmsnorm_rope_pool_kernel(RopeArgs a, int blk, int nb, float *pq,
                                                                    float *pk) {
   static_assert(kHeadsPerWave % 4 == 0, "four 16-lane groups per wave");
@@ -211,7 +220,7 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_pool_kernel(RopeArgs a, i
   auto token_of = [&](int n) __attribute__((always_inline)) { return r0 + wave + 4 * (n < mine ? n : mine - 1); };
   auto load = [&](Token &in, int n) __attribute__((always_inline)) {
     const int s = token_of(n);
-    load_rope(in.R, a.rope + b * a.rsb + s * a.rss, c, nh);
+    load_rope<kRot128>(in.R, a.rope + b * a.rsb + s * a.rss, c, nh);
     const uint16_t *qrow = a.q + b * a.qsb + s * a.qss + c * 8;
     const uint16_t *krow = a.k + b * a.ksb + s * a.kss + c * 8;
 #pragma unroll
@@ -230,8 +239,8 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_pool_kernel(RopeArgs a, i
       float xq[8], xk[8];
       unpack8(in.q[i], xq);
       unpack8(in.k[i], xk);
-      norm_rope_row(xq, wq, a.eps, in.R, c, nh);
-      norm_rope_row(xk, wk, a.eps, in.R, c, nh);
+      norm_rope_row<kRot128>(xq, wq, a.eps, in.R, c, nh);
+      norm_rope_row<kRot128>(xk, wk, a.eps, in.R, c, nh);
       const u32x4 oq = pack8(xq), ok = pack8(xk);
       if (heads[i] < a.H) {
         *(u32x4 *)(qrow + heads[i] * a.qsh) = oq;
@@ -305,15 +314,27 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_pool_kernel(RopeArgs a, i
 // and 490 / 655 at H=56 S=42120 (4613), where 2 KiB per access of a token's q or k
 // against 1 KiB decides.
 constexpr int64_t kPoolWideWgs = 256;
+// With rot = 128 the row needs no branches, and from four workgroups per CU on the
+// 8-head form keeps two tokens in flight (its registers hold fewer workgroups on
+// a CU, which a launch of one or two rounds feels): one token and branches / two
+// tokens without, H=28 S=42120 (1756 workgroups) 269.7 / 265.6 us, H=56 S=24000 in
+// blocks of 128 (1316) 324 / 316, but H=28 S=10000 (420) 72.3 / 75.0 and H=28 S=8192
+// (512) 55.4 / 56.4.  4 heads, with branches / without: 28.1 / 24.7 us at H=14
+// S=4104, 21.0 / 19.4 at H=4 S=1024.
+constexpr int64_t kPoolDeepWgs = 1024;
 int launch_qk_rmsnorm_rope_pool(const RopeArgs &a, int blk, float *pq, float *pk, hipStream_t s) {
   const int nb = (a.S + blk - 1) / blk;
-  const int64_t blocks = (int64_t)a.B * nb;
-  if (blocks * ((a.H + 7) / 8) < kPoolWideWgs)
-    hipLaunchKernelGGL((qk_rmsnorm_rope_pool_kernel<4, 2>), dim3((unsigned)(blocks * ((a.H + 3) / 4))), dim3(256),
-                       0, s, a, blk, nb, pq, pk);
-  else
-    hipLaunchKernelGGL((qk_rmsnorm_rope_pool_kernel<8, 1>), dim3((unsigned)(blocks * ((a.H + 7) / 8))), dim3(256),
-                       0, s, a, blk, nb, pq, pk);
+  const int64_t blocks = (int64_t)a.B * nb, wide = blocks * ((a.H + 7) / 8);
+  const bool full = a.rot == kRopeD;
+  auto *kernel = qk_rmsnorm_rope_pool_kernel<8, 1, false>;
+  int64_t wgs = wide;
+  if (wide < kPoolWideWgs) {
+    kernel = full ? qk_rmsnorm_rope_pool_kernel<4, 2, true> : qk_rmsnorm_rope_pool_kernel<4, 2, false>;
+    wgs = blocks * ((a.H + 3) / 4);
+  } else if (full && wide >= kPoolDeepWgs) {
+    kernel = qk_rmsnorm_rope_pool_kernel<8, 2, true>;
+  }
+  hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256), 0, s, a, blk, nb, pq, pk);
   return check_launch("qk_rmsnorm_rope_pool_kernel");
 }
 
@@ -321,16 +342,16 @@ int launch_qk_rmsnorm_rope(const RopeArgs &a, hipStream_t s) {
   const int hpw = rope_heads_per_wave(a.H);
   const int64_t items = (int64_t)a.B * a.S * ((a.H + hpw - 1) / hpw);
   const int64_t blocks = (items + 3) / 4;
-  if (hpw == 28)
-    hipLaunchKernelGGL(qk_rmsnorm_rope_kernel<28>, dim3((unsigned)blocks), dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL(qk_rmsnorm_rope_kernel<16>, dim3((unsigned)blocks), dim3(256), 0, s, a);
+  const bool full = a.rot == kRopeD;
+  auto *kernel = hpw == 28 ? (full ? qk_rmsnorm_rope_kernel<28, true> : qk_rmsnorm_rope_kernel<28, false>)
+                           : (full ? qk_rmsnorm_rope_kernel<16, true> : qk_rmsnorm_rope_kernel<16, false>);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, s, a);
   return check_launch("qk_rmsnorm_rope_kernel");
 }
 
 int rope_kernel_attrs(double out[6]) {
   hipFuncAttributes fa;
-  const void *fn = reinterpret_cast<const void *>(&qk_rmsnorm_rope_kernel<28>);  // the H=56 width
+  const void *fn = reinterpret_cast<const void *>(&qk_rmsnorm_rope_kernel<28, true>);  // the H=56 width
   if (hipFuncGetAttributes(&fa, fn) != hipSuccess) return fail(H3A_ERR_HIP, "hipFuncGetAttributes failed");
   int blocks = 0, dev = 0, clk = 0, max_threads = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, fn, 256, 0) != hipSuccess ||

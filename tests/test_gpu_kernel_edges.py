@@ -67,7 +67,8 @@ def test_tile_lut_chunk_and_slice_edges(gpu, blk_q, blk_k, Sq, Skv):
 
 
 @pytest.mark.parametrize("S,H,blk,rot", [(63, 3, 64, 128), (64, 4, 64, 64), (65, 8, 64, 128), (1, 1, 64, 128),
-                                         (130, 14, 48, 96), (4104, 56, 64, 128), (2100, 60, 16, 32)])
+                                         (130, 14, 48, 96), (4104, 56, 64, 128), (2100, 60, 16, 32),
+                                         (2100, 60, 16, 128)])
 def test_pooled_prologue_tokens_heads_edges(gpu, S, H, blk, rot):
     """The pooling prologue in 4-head and 8-head workgroups, ragged heads and last blocks of fewer tokens
     than waves: its rows and means equal the plain prologue's and block_pool's bit for bit."""
