@@ -92,7 +92,8 @@ int h3a_attn_fwd(const void *q, const void *k, const void *v, void *o,
  * floating-point rounding.  Problems of four or more rounds of tiles also
  * run on a persistent grid whose workgroups take tiles from per-XCD work
  * queues (1 KiB of counters in the workspace, cleared by the call itself
- * with a kernel before the attention launch).  h3a_attn_fwd_workspace_size
+ * with a kernel before the attention launch), and problems of few tiles may
+ * run on shorter ones.  h3a_attn_fwd_workspace_size
  * gives the bytes needed for a problem on the current device (0: nothing is
  * split or queued, and workspace may be NULL).  The workspace must stay untouched until the call's
  * work on `stream` has completed, and two calls in flight at once need two
