@@ -745,7 +745,8 @@ struct QTile {
 // s0 + x, s0 + x + 2, ... of the range, so that with kKeySplit every 32-row slice
 // is spread over four waves, otherwise over two; after the loop they exchange
 // their parts through LDS, each wave merging and storing its share of the dims.
-template <class L, int NSUB, bool kSparse, bool kKeySplit, bool kWideKV, bool kTileMask, bool kHalves>
+// kHalfLut: the same over the stages of the block's LUT row instead of all keys.
+template <class L, int NSUB, bool kSparse, bool kKeySplit, bool kWideKV, bool kTileMask, bool kHalves, bool kHalfLut>
 __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item, const bool remapped,
                                               PingPongLds<L, NSUB, kSparse> &lds, PhaseClock &pc) {
   constexpr int NW = 8;
@@ -757,6 +758,8 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
   static_assert(!kKeySplit || (kSparse && NSUB == 2), "key-split pairs are block-sparse, 64-key stages");
   static_assert(!kTileMask || kKeySplit, "tile masks run on the key-split pairs");
   static_assert(!kHalves || (kSparse && !kTileMask), "key halves run on the pairs kernels");
+  static_assert(!kHalfLut || kHalves, "LUT halves are key halves");
+  constexpr bool kLut = kSparse && (!kHalves || kHalfLut);  // stages come from a LUT row
   auto &kbuf_all = lds.k;
   auto &vbuf_all = lds.v;
 
@@ -855,7 +858,7 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
   // own column: its fetch, scores and mask).  ntile is the row's entry count.
   int ntile = 0;
   const uint32_t smag = stage_magic(a.sub);  // block_of_stage_magic(t, smag) = t / a.sub
-  if constexpr (kHalves) {
+  if constexpr (kHalves && !kHalfLut) {
     j0 = split_part < 0 ? 0 : (int)((int64_t)nstages * split_part / a.split_pieces);
     const int len = (split_part < 0 ? nstages : (int)((int64_t)nstages * (split_part + 1) / a.split_pieces)) - j0;
     ngrp = (len + 1 - grp) / 2;  // this group's stages: j0 + grp + 2j
@@ -878,7 +881,7 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
     lut_row = a.lut + ((int64_t)bh * a.nqb + (qb < a.nqt ? qb : 0) / a.qmul) * a.lut_stride;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int e = kTileMask ? 2 * j + kh : block_of_stage_magic(j, smag);
+      const int e = kTileMask ? 2 * j + kh : block_of_stage_magic(kHalfLut ? 2 * j + grp : j, smag);
       e_pre[j] = ((ConstInts)lut_row)[e < a.lut_stride ? e : a.lut_stride - 1];
     }
     auto stages_of = [&](int qb, int cnt) __attribute__((always_inline)) -> int {
@@ -900,7 +903,13 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
     ngrp = part_of(stages_of(qb, cnt_own), gj0);
     const int nother = part_of(stages_of(qo, cnt_oth), other_j0);
     niter = ngrp > nother ? ngrp : nother;
+    if constexpr (kHalfLut) {  // (unsplit) both groups read one row: its stages grp, grp + 2, ...
+      niter = (ngrp + 1) / 2;
+      ngrp = (ngrp + 1 - grp) / 2;
+    }
   }
+  // List stage of this group's stage j.
+  auto list_stage = [&](int j) __attribute__((always_inline)) -> int { return kHalfLut ? 2 * j + grp : gj0 + j; };
   // Sparse: LUT entry of local stage j (a key block of a.sub stages; read
   // through the constant address space, so it is a scalar load), and the
   // stage's first key from it.  Past this group's last stage, and for LUT
@@ -910,7 +919,7 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
   // group's part of the row (entry 0 for an empty list, whose keys are all
   // Skv whatever the entry).
   auto lut_entry = [&](int j) __attribute__((always_inline)) -> int {
-    if constexpr (kSparse && !kHalves) {
+    if constexpr (kLut) {
       const __attribute__((address_space(4))) int32_t *row =
           (const __attribute__((address_space(4))) int32_t *)lut_row;
       const int jc = j < ngrp ? j : ngrp - 1;
@@ -918,7 +927,7 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
         const int i = 2 * (jc > 0 ? jc : 0) + kh;
         return row[i < a.lut_stride ? i : a.lut_stride - 1];
       } else {
-        return row[block_of_stage_magic(gj0 + (jc > 0 ? jc : 0), smag)];
+        return row[block_of_stage_magic(list_stage(jc > 0 ? jc : 0), smag)];
       }
     } else {
       return 0;
@@ -929,15 +938,15 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
   // entry negative, so it still names no key block.  Past the row's entries
   // (the last stage can hold one column) the key is Skv.
   auto key_of_entry = [&](int j, int e) __attribute__((always_inline)) -> int {
-    if constexpr (kHalves) {
+    if constexpr (kHalves && !kHalfLut) {
       return j < ngrp ? (j0 + grp + 2 * j) * BN : a.Skv;
     } else if constexpr (kSparse) {
       const int kb = kTileMask ? (e >> 8) : e;
       // Two equivalent forms; each measured faster in one kernel (the
       // arithmetic one +0.5 % in the 128-row pairs, the select one +0.6 % in
       // the key-split pairs), through the code layout around them.
-      const int key0 = kKeySplit ? lut_stage_key0_sel(gj0 + j, kb, a.nkb, a.blk_k, a.sub, smag, a.Skv)
-                                 : lut_stage_key0_magic(gj0 + j, kb, a.nkb, a.blk_k, a.sub, smag, a.Skv);
+      const int key0 = kKeySplit ? lut_stage_key0_sel(list_stage(j), kb, a.nkb, a.blk_k, a.sub, smag, a.Skv)
+                                 : lut_stage_key0_magic(list_stage(j), kb, a.nkb, a.blk_k, a.sub, smag, a.Skv);
       if constexpr (kTileMask) return j < ngrp && 2 * j + kh < ntile ? key0 : a.Skv;
       else return j < ngrp ? key0 : a.Skv;
     } else {
@@ -947,11 +956,11 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
   auto key_base = [&](int j) __attribute__((always_inline)) -> int { return key_of_entry(j, lut_entry(j)); };
   // The same for the prologue's stages 0-3, from the entries loaded up front.
   auto pro_entry = [&](int j) __attribute__((always_inline)) -> int {
-    if constexpr (kSparse && !kHalves) return split_part < 0 ? e_pre[j] : lut_entry(j);
+    if constexpr (kLut) return split_part < 0 ? e_pre[j] : lut_entry(j);
     else return 0;
   };
   auto pro_key = [&](int j) __attribute__((always_inline)) -> int { return key_of_entry(j, pro_entry(j)); };
-  if (kSparse && !kHalves && niter == 0) {
+  if (kLut && niter == 0) {
     // Neither query block of the pair keeps a key block (in this piece): O = 0,
     // or an empty partial result (m = -inf, l = 0, O = 0).
     if (piece >= 0) {
@@ -965,7 +974,7 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
       }
       return;
     }
-    if (qrow < a.Sq && kh == 0) {
+    if (qrow < a.Sq && kh == 0 && (!kHalfLut || grp == 0)) {
       uint16_t *p = Ob + (int64_t)qrow * a.oss + 4 * g;
 #pragma unroll
       for (int c = 0; c < 16; ++c) *(u32x2 *)(p + 8 * c) = u32x2{0, 0};
@@ -1459,7 +1468,7 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
 }
 
 template <class L, int NSUB, bool kSparse = false, bool kKeySplit = false, bool kWideKV = false,
-          bool kTileMask = false, bool kHalves = false>
+          bool kTileMask = false, bool kHalves = false, bool kHalfLut = false>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 attn_fwd_pingpong_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(16))) PingPongLds<L, NSUB, kSparse> lds;
@@ -1501,7 +1510,7 @@ attn_fwd_pingpong_kernel(AttnArgs a) {
       if (item < 0) break;
     }
     pc.begin(blockIdx.x == 0);
-    pingpong_item<L, NSUB, kSparse, kKeySplit, kWideKV, kTileMask, kHalves>(args, item, args.sched != nullptr, lds, pc);
+    pingpong_item<L, NSUB, kSparse, kKeySplit, kWideKV, kTileMask, kHalves, kHalfLut>(args, item, args.sched != nullptr, lds, pc);
     KernargPtr kq = (KernargPtr)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(kq));
     if (!kq->sched) break;
@@ -1898,7 +1907,20 @@ int plan_attn_split(int B, int H, int Sq, int Skv, SplitPlan *plan) {
 int plan_attn_sparse_split(int B, int H, int Sq, int blk_q, int blk_k, int max_k_blocks, SplitPlan *plan) {
   const int rows = sparse_sub_block_rows(blk_q);
   const int64_t nsub = (Sq + rows - 1) / rows;
-  return plan_tiles((int64_t)B * H * ((nsub + 1) / 2), max_k_blocks * (blk_k / 64), rows == 128, true, plan);
+  const int rc =
+      plan_tiles((int64_t)B * H * ((nsub + 1) / 2), max_k_blocks * (blk_k / 64), rows == 128, true, plan);
+  if (rc || rows == 128) return rc;
+  // 64-row blocks that all fit on the chip one per CU: a workgroup each, its two
+  // groups on alternate stages of the block's list, half as long as a pair's.
+  // Pairs / one block each: 52 / 26 us at 1 head of S=10000 keeping 39 blocks,
+  // 19.5 / 14.8 at 4 of S=4000 keeping 9, 17 / 14.5 at 4 of S=2000 keeping 11; lists
+  // of fewer than 8 stages gain nothing over the four-way merge (14 heads of S=1024
+  // keeping 5: 13 / 14).
+  int cus = 0;
+  const int rc_cus = device_cu_count(&cus);
+  if (rc_cus) return rc_cus;
+  if ((int64_t)B * H * nsub <= cus && max_k_blocks * (blk_k / 64) >= 8) plan->rows = 64;
+  return H3A_OK;
 }
 
 // The same for a tile LUT (64-row sub-blocks, unsplit): max_tiles entries
@@ -2023,6 +2045,14 @@ int launch_attn_sparse_split(const AttnArgs &a, int blk_q, const SplitPlan &plan
     const int rc = check_launch("tile_pair_map_kernel");
     if (rc) return rc;
     p.pair_map = map;
+  }
+  if (!tiles && plan.rows == 64) {  // one block per workgroup (plan_attn_sparse_split)
+    p.total = a.B * a.H * a.nqt;
+    const PingPongKernel one =
+        wide_kv(a) ? attn_fwd_pingpong_kernel<SwzLayout, kStageSub, true, true, true, false, true, true>
+                   : attn_fwd_pingpong_kernel<SwzLayout, kStageSub, true, true, false, false, true, true>;
+    hipLaunchKernelGGL(one, dim3(p.total), dim3(512), 0, s, p);
+    return check_launch("attn_fwd_pingpong_kernel<sparse, one block>");
   }
   if (plan.pieces < 2 && !plan.dynamic) return launch_attn_sparse(p, blk_q, s, tiles);
   const int rows = tiles ? 64 : sparse_sub_block_rows(blk_q);

@@ -80,7 +80,7 @@ struct SplitPlan {
   bool dynamic; // persistent grid with per-XCD work queues
   size_t sched_off;  // byte offset of the queue counters in the workspace
   bool pair_map;     // tile path: sub-blocks paired by stage count (map at offset 0)
-  int rows;          // dense: tile height (256, 128 or 64)
+  int rows;          // dense: tile height (256, 128 or 64); block-sparse: 64 for one 64-row block per workgroup
 };
 
 // Launchers implemented in h3a_attn.hip / h3a_prologue.hip.

@@ -273,11 +273,10 @@ def attn_fwd_blocksparse(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, lut:
             *st, lut.data_ptr(), counts.data_ptr(),
             int(blk_q), int(blk_k), int(lut.shape[3]), sc)
     with _on_device(q):
-        nbytes = (sparse_workspace_bytes(B, H, Sq, Skv, blk_q, blk_k, int(lut.shape[3]), D)
-                  if split_tail else 0)
-        if nbytes:
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
-            rc = lib().h3a_attn_fwd_blocksparse_ws(*args, ws.data_ptr(), nbytes, _stream(q))
+        if split_tail:
+            nbytes = sparse_workspace_bytes(B, H, Sq, Skv, blk_q, blk_k, int(lut.shape[3]), D)
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+            rc = lib().h3a_attn_fwd_blocksparse_ws(*args, ws.data_ptr() if nbytes else None, nbytes, _stream(q))
             check("h3a_attn_fwd_blocksparse_ws", rc)
         else:
             rc = lib().h3a_attn_fwd_blocksparse(*args, _stream(q))

@@ -148,3 +148,24 @@ def test_block_select_rows_per_workgroup(gpu, H, nq, nk):
     assert torch.equal(cnt.cpu(), want.sum(3, dtype=torch.int32))
     idx = torch.where(want.bool(), torch.arange(nk), nk).sort(3).values[..., :lut.shape[3]]
     assert torch.equal(lut.cpu(), torch.where(idx < nk, idx, -1).int())
+
+
+@pytest.mark.parametrize("H,blk_q,blk_k,Sq,Skv", [(1, 64, 64, 64, 64), (2, 64, 64, 333, 1000), (3, 64, 128, 1000, 1090),
+                                                  (2, 64, 256, 640, 2500), (2, 192, 64, 700, 1100),
+                                                  (4, 192, 192, 4096, 777), (5, 64, 64, 4096, 333)])
+def test_one_sparse_block_per_workgroup(gpu, H, blk_q, blk_k, Sq, Skv):
+    """64-row query blocks, few enough for one per CU (and, last, just too many): both groups on one block's
+    list, with empty, one-entry and full lists, against the masked oracle."""
+    rng = np.random.default_rng(Sq + Skv)
+    q, k, v = (randn_bf16(rng, (1, H, n, 128)) for n in (Sq, Skv, Skv))
+    bmap = (rng.random((1, H, -(-Sq // blk_q), -(-Skv // blk_k))) < 0.4).astype(np.uint8)
+    bmap[0, 0, 0] = 0
+    bmap[0, -1, -1] = 1
+    bmap[0, :, -2:-1] = 0
+    bmap[0, :, -2:-1, -1] = 1
+    lut, cnt = h3attn.block_map_to_lut(torch.from_numpy(bmap).to(gpu))
+    out = torch.full((1, Sq, H, 128), float("nan"), dtype=torch.bfloat16, device=gpu).transpose(1, 2)
+    ops.attn_fwd_blocksparse(*(to_dev_bf16(x, gpu) for x in (q, k, v)), lut, cnt, blk_q, blk_k, out=out)
+    got = oracle.bf16_to_f32(from_dev_bf16(out)).reshape(out.shape)
+    assert_close_absmax(got, oracle.attn_fwd(q, k, v, block_map=bmap, blk_q=blk_q, blk_k=blk_k),
+                        what=f"{H} heads {blk_q}x{blk_k}")
