@@ -1852,19 +1852,28 @@ constexpr int kCombineCycles = 9000, kCombineCyclesPerMB = 1000;
 // 18.8; H=14 S=1000 23.1 / 18.8 / 14.0; H=28 S=700 18.3 / 17.0 / 24.3; H=4 S=8000
 // 125.3 / 120.7 / 137.0; H=14 S=3000 64.5 / 77.5 / 80.5; H=56 S=2000 108.6 / 130.5 /
 // 148.7; the choice is within 0.6 us of the least in each.
+//
+// Whether a call needs a workspace at all does not depend on the form: a launch
+// whose 256-row tiles would be neither split nor queued needs none, so its
+// shorter forms are not either (one head of S=33000 would run 128-row tiles in
+// ranges otherwise), and one whose 256-row tiles would be asks for
+// kMinWorkspace even where the form that runs writes nothing there.
 int plan_attn_split(int B, int H, int Sq, int Skv, SplitPlan *plan) {
   int cus = 0;
   int rc = device_cu_count(&cus);
   if (rc) return rc;
+  constexpr size_t kMinWorkspace = 256;
   const int stages = (Skv + kBN - 1) / kBN;
   int64_t best = -1;
-  bool splits = false;
+  bool bare = false;  // no workspace
   for (const DenseForm &f : kDenseForms) {
     const int64_t tiles = (int64_t)B * H * (((int64_t)Sq + f.rows - 1) / f.rows);
     if (tiles > INT_MAX && f.rows != 256) continue;
     SplitPlan p;
-    rc = plan_tiles(tiles, stages, true, true, &p);
+    rc = plan_tiles(tiles, stages, !bare, true, &p);
     if (rc) return rc;
+    if (f.rows == 256) bare = p.bytes == 0;
+    if (bare && p.bytes > 0) continue;
     // Cycles of a round of items of n stages on `busy` CUs, in cycles of a full
     // chip's clock: the power limit holds 256 busy CUs at about 1.7 GHz, and
     // fewer run faster, up to 2.35 GHz (72 % of the time) at 184 CUs and less.
@@ -1875,7 +1884,6 @@ int plan_attn_split(int B, int H, int Sq, int Skv, SplitPlan *plan) {
     };
     const int64_t r = tiles % cus, full = tiles / cus * pass(stages, cus);
     int64_t cost = full + (r ? pass(stages, r) : 0);
-    splits = splits || p.pieces >= 2;
     if (p.pieces >= 2) {
       int pieces = 1;
       for (int n = 2; n <= p.pieces; ++n) {
@@ -1896,9 +1904,7 @@ int plan_attn_split(int B, int H, int Sq, int Skv, SplitPlan *plan) {
       *plan = p;
     }
   }
-  // A launch that some form would split asks for a workspace, so that a caller
-  // prepared for one does not depend on the form.
-  if (splits && plan->bytes == 0) plan->bytes = 256;
+  if (!bare && plan->bytes == 0) plan->bytes = kMinWorkspace;
   return H3A_OK;
 }
 

@@ -104,7 +104,7 @@ def _prepare_attn(q, k, v, out):
 
 
 def attn_workspace_bytes(B: int, H: int, Sq: int, Skv: int, D: int = HEAD_DIM) -> int:
-    """Workspace bytes h3a_attn_fwd_ws needs on the current device (0: no split)."""
+    """Workspace bytes h3a_attn_fwd_ws needs on the current device (0: none)."""
     n = ctypes.c_size_t(0)
     check("h3a_attn_fwd_workspace_size", lib().h3a_attn_fwd_workspace_size(B, H, Sq, Skv, D, ctypes.byref(n)))
     return int(n.value)

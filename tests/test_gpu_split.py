@@ -134,3 +134,67 @@ def test_queued_dispatch_with_split_tail(gpu):
                         what="queued split heads vs oracle")
     whole = oracle.bf16_to_f32(from_dev_bf16(o_whole[:, H - 2:].contiguous())).reshape(1, 2, Sq, 128)
     assert_close_absmax(got, whole, what="queued split vs unsplit")
+
+
+def _whole_tiles_need(B, H, Sq, Skv):
+    """Whether 256-row tiles would be split (ranges of at least 4 of the 64-key stages) or queued."""
+    cus, tiles, stages = _cus(), B * H * -(-Sq // 256), -(-Skv // 64)
+    r = tiles % cus
+    return tiles >= 4 * cus or (r > 0 and min(cus // r, stages // 4) >= 2)
+
+
+@pytest.mark.parametrize("B,H,Sq,Skv", [(2, 14, 1160, 4104), (1, 14, 3000, 3000), (1, 56, 2000, 2000),
+                                        (1, 1, 33000, 33000), (1, 4, 8202, 36179), (1, 2, 300, 300)])
+def test_no_workspace_where_whole_tiles_need_none(gpu, B, H, Sq, Skv):
+    """Whether a call needs a workspace does not depend on the tile height that runs: NULL is
+    accepted (and the result that of the unsplit tiles) where 256-row tiles are neither split nor
+    queued on 256 CUs, also where shorter tiles could be."""
+    if _whole_tiles_need(B, H, Sq, Skv):
+        pytest.skip("split on this device's CU count")
+    assert ops.attn_workspace_bytes(B, H, Sq, Skv) == 0
+    g = torch.Generator(device=gpu).manual_seed(Sq)
+    q, k, v = (torch.randn(B, H, n, 128, generator=g, device=gpu, dtype=torch.bfloat16) for n in (Sq, Skv, Skv))
+    o = torch.full_like(q, float("nan"))
+    L, st = h3attn._lib.lib(), [h3attn._lib.strides3(*t.stride()[:3]) for t in (q, k, v, o)]
+    assert L.h3a_attn_fwd_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), B, H, Sq, Skv, 128, *st,
+                             1.0 / np.sqrt(128), None, 0, ops._stream(q)) == 0, L.h3a_last_error()
+    want = ops.attn_fwd(q, k, v, split_tail=False).float()
+    d = (o.float() - want).abs()
+    # both round O and every p to bf16 (see test_short_tiles_and_key_ranges_match_whole_tiles)
+    assert d.max() <= 1e-2 * want.abs().max() and d.mean() <= 2.0 ** -7 * want.abs().mean()
+
+
+def test_workspace_need_over_a_range_of_problems(gpu):
+    rng = np.random.default_rng(3)
+    for _ in range(4000):
+        B, H = int(rng.choice([1, 1, 2, 4, 32])), int(rng.integers(1, 57))
+        Sq, Skv = (int(np.exp(rng.uniform(0, np.log(42120)))) for _ in range(2))
+        need = ops.attn_workspace_bytes(B, H, Sq, Skv)
+        assert (need > 0) == _whole_tiles_need(B, H, Sq, Skv), (B, H, Sq, Skv, need)
+
+
+@pytest.mark.parametrize("B,H,Sq,Skv,rows", [(1, 1, 64, 2000, 64), (32, 9, 23, 1007, 64), (2, 29, 69, 4207, 128),
+                                             (32, 9, 74, 764, 128), (2, 32, 197, 6423, 256), (4, 33, 457, 457, 256)])
+def test_split_partials_of_every_tile_height(gpu, B, H, Sq, Skv, rows):
+    """Problems whose tail is split at each tile height, alone and after a whole round: the workspace
+    is the partials of the last round's r tiles in 2 or more ranges (per row 128 sums, a max and a
+    row sum), the call writes there and no further, and the result matches the oracle."""
+    cus, tiles = _cus(), B * H * -(-Sq // rows)
+    if cus != 256:
+        pytest.skip("the shapes are chosen for 256 CUs")
+    need = ops.attn_workspace_bytes(B, H, Sq, Skv)
+    r = tiles % cus
+    pieces, rest = divmod(need, r * rows * 130 * 4)
+    assert rest == 0 and 2 <= pieces <= cus // r, "this shape is meant to exercise the split"
+    rng = np.random.default_rng(Sq + Skv)
+    q, k, v = (randn_bf16(rng, (B, H, n, 128)) for n in (Sq, Skv, Skv))
+    qd, kd, vd = (to_dev_bf16(x, gpu) for x in (q, k, v))
+    o = torch.full_like(qd, float("nan"))
+    ws = torch.full((need + 4096,), 0x7F, dtype=torch.uint8, device=gpu)
+    _ws_call(qd, kd, vd, o, ws)
+    assert torch.all(ws[need:] == 0x7F) and not torch.any(ws[:need].view(torch.int32) == 0x7F7F7F7F)
+    last = (slice(B - 1, B), slice(H - 1, H))  # the split tiles are the last ones
+    got = oracle.bf16_to_f32(from_dev_bf16(o[last].contiguous())).reshape(1, 1, Sq, 128)
+    assert_close_absmax(got, oracle.attn_fwd(q[last], k[last], v[last]), what=f"{rows}-row tiles in {pieces} ranges")
+    d = (o.float() - ops.attn_fwd(qd, kd, vd, split_tail=False).float()).abs()
+    assert d.max() <= 1e-2 * o.float().abs().max()
