@@ -1829,29 +1829,35 @@ static int plan_tiles(int64_t tiles, int stages, bool splittable, bool queued, S
   return H3A_OK;
 }
 
-// Dense tile heights and what they cost in shader cycles (phase profile, whole
-// chip busy): a pair of 64-key stages, and an item's prologue and epilogue.
-// 256 rows share one K/V stream and run 4-5 % more rows per cycle than two
-// 128-row tiles, whose groups each fetch their own; 64 rows cost 38 % more per
-// row again.  But a launch of few tiles leaves CUs idle or cuts them into many
-// key ranges, each with its own prologue and 520 bytes of partial sums a row: at
-// 128 or 64 rows there are more, shorter items instead.
+// Dense tile heights and what they cost, in shader cycles of a full chip's clock:
+// `group` 64-key stages (128- and 64-row tiles take theirs in pairs, one per wave
+// group, so an odd last stage takes as long as a pair), and an item's ends.  256
+// rows share one K/V stream; 128-row tiles, whose groups each fetch their own,
+// take 4 to 10 % longer in launches of many rounds and have partial results to
+// merge; 64 rows cost 19 % more per row again.  But a launch of few tiles leaves
+// CUs idle or cuts them into many key ranges, each with its own prologue and 520
+// bytes of partial sums a row: at 128 or 64 rows there are more, shorter items
+// instead.  Fitted to 400 problems of up to 1800 heads, 60 .. 42000 rows and keys,
+// each timed at every height and up to 12 numbers of ranges: the choice is 0.8 %
+// off the best on average and no slower than 256-row tiles in CUs / r ranges.
 struct DenseForm {
-  int rows, pair_cycles, item_cycles;
+  int rows, group, group_cycles, item_cycles;
 };
-constexpr DenseForm kDenseForms[] = {{256, 2 * 2567, 13000}, {128, 2860, 12000}, {64, 1980, 10000}};
-// The combine: a launch's latency, and its reads and the partials' writes at
-// about 1000 cycles a megabyte (35 MB: 8.6 us to read, about 7 to write).
-constexpr int kCombineCycles = 9000, kCombineCyclesPerMB = 1000;
+constexpr DenseForm kDenseForms[] = {{256, 1, 2600, 7000}, {128, 2, 2860, 11500}, {64, 2, 1700, 8000}};
+// The combine: a launch's latency, and its reads and the partials' writes by the
+// megabyte.
+constexpr int kCombineCycles = 8500, kCombineCyclesPerMB = 600;
 
 // The form and the number of key ranges of the tail with the least estimated
 // time: whole rounds of tiles, then the last round's r tiles in P ranges each
 // (P = 1 .. CUs / r with at least kMinSplitStages stages per range; at least 2
-// after a whole round, where the combine is a small part of the launch).  Measured per call, 256 / 128 / 64 rows (one
-// card, graph replay): H=2 S=300 11.0 / 11.5 / 8.6 us; H=4 S=2048 26.5 / 26.8 /
-// 18.8; H=14 S=1000 23.1 / 18.8 / 14.0; H=28 S=700 18.3 / 17.0 / 24.3; H=4 S=8000
-// 125.3 / 120.7 / 137.0; H=14 S=3000 64.5 / 77.5 / 80.5; H=56 S=2000 108.6 / 130.5 /
-// 148.7; the choice is within 0.6 us of the least in each.
+// after a whole round, where the combine is a small part of the launch).  Measured
+// per call, 256 / 128 / 64 rows: H=2 S=300 11.0 / 11.5 / 8.6 us; H=4 S=2048 26.5 /
+// 26.8 / 18.8; H=14 S=1000 23.1 / 18.8 / 14.0; H=28 S=700 18.3 / 17.0 / 24.3; H=4
+// S=8000 125.3 / 120.7 / 137.0; H=14 S=3000 64.5 / 77.5 / 80.5; H=56 S=2000 108.6 /
+// 130.5 / 148.7; and over more than one round, B=8 H=56 Sq=128 Skv=1000 53.9 / 46.9 /
+// 59.0, B=32 H=14 Sq=97 Skv=108 16.4 / 18.9 / 25.4, B=32 H=14 S=475 88.8 / 99.1 / 126.2,
+// H=52 Sq=2860 Skv=1003 88.2 / 93.7 / 114.1.
 //
 // Whether a call needs a workspace at all does not depend on the form: a launch
 // whose 256-row tiles would be neither split nor queued needs none, so its
@@ -1878,7 +1884,7 @@ int plan_attn_split(int B, int H, int Sq, int Skv, SplitPlan *plan) {
     // chip's clock: the power limit holds 256 busy CUs at about 1.7 GHz, and
     // fewer run faster, up to 2.35 GHz (72 % of the time) at 184 CUs and less.
     auto pass = [&](int n, int64_t busy) -> int64_t {
-      const int64_t cycles = (int64_t)(n + 1) / 2 * f.pair_cycles + f.item_cycles;
+      const int64_t cycles = ((int64_t)n + f.group - 1) / f.group * f.group_cycles + f.item_cycles;
       const int64_t pct = 100 * busy / cus;
       return cycles * (pct < 72 ? 72 : pct) / 100;
     };

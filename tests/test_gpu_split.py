@@ -198,3 +198,21 @@ def test_split_partials_of_every_tile_height(gpu, B, H, Sq, Skv, rows):
     assert_close_absmax(got, oracle.attn_fwd(q[last], k[last], v[last]), what=f"{rows}-row tiles in {pieces} ranges")
     d = (o.float() - ops.attn_fwd(qd, kd, vd, split_tail=False).float()).abs()
     assert d.max() <= 1e-2 * o.float().abs().max()
+
+
+@pytest.mark.parametrize("B,H,Sq,Skv", [(32, 14, 97, 108), (16, 56, 100, 300), (32, 56, 64, 64)])
+def test_many_short_items_run_on_whole_tiles(gpu, B, H, Sq, Skv):
+    """More than a round of tiles with few keys each: 256-row tiles, whose ends cost the least, run
+    unsplit, so the result is h3a_attn_fwd's bit for bit."""
+    if _cus() != 256:
+        pytest.skip("the shapes are chosen for 256 CUs")
+    g = torch.Generator(device=gpu).manual_seed(Sq)
+    q, k, v = (torch.randn(B, H, n, 128, generator=g, device=gpu, dtype=torch.bfloat16) for n in (Sq, Skv, Skv))
+    assert torch.equal(ops.attn_fwd(q, k, v), ops.attn_fwd(q, k, v, split_tail=False))
+
+
+def test_tail_ranges_where_short_tiles_are_no_gain(gpu):
+    """2.4 rounds of 256-row tiles of 16 stages: the tail's 112 tiles in two ranges, not queued 128-row tiles."""
+    if _cus() != 256:
+        pytest.skip("the shape is chosen for 256 CUs")
+    assert ops.attn_workspace_bytes(1, 52, 2860, 1003) == 112 * 2 * 256 * 130 * 4
