@@ -709,8 +709,12 @@ struct PingPongLds {
 // before and after: key-split pairs 11.9k -> 7.0k ticks (H=56 S=10000), 128-row
 // pairs 13.3k -> 9.3k, dense 11.5k -> 10.9k (its 64 KiB of query rows per item
 // come from HBM and set the pace), 8.5k -> 6.1k where they come from L2.
-// Rows past Sq repeat the last row (64-bit addresses: no limit on the stride);
-// what becomes of them is never stored.
+// Rows past Sq fetch the last row (64-bit addresses: no limit on the stride);
+// what becomes of them is never stored.  The dense kernel reads them as zeros,
+// whose products cost no switching power, which sets the clock: 86.9 -> 84.5 us at
+// B=8 H=28 Sq=130 Skv=3000, 54.4 -> 53.0 at B=4 H=56 Sq=300 Skv=1000.  The others, with
+// fewer rows to a tile, take longer for the selects than they save (14 heads of
+// S=4104 in 128x128 blocks 42.0 -> 42.8).
 template <class L>
 struct QTile {
   static_assert(L::kKRow == 256 && L::kKSlots == 16, "one K row per query row");
@@ -728,10 +732,13 @@ struct QTile {
       m0 = opaque_sadd<1024u>(m0);
     }
   }
-  __device__ __forceinline__ static void read(u32x4 (&qf)[8], const uint16_t *tile, int k_rd) {
+  // `live`: false reads zeros.
+  __device__ __forceinline__ static void read(u32x4 (&qf)[8], const uint16_t *tile, int k_rd, bool live) {
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks)
-      qf[ks] = *(const u32x4 *)(reinterpret_cast<const char *>(tile) + L::k_off(k_rd, ks));
+    for (int ks = 0; ks < 8; ++ks) {
+      const u32x4 v = *(const u32x4 *)(reinterpret_cast<const char *>(tile) + L::k_off(k_rd, ks));
+      qf[ks] = live ? v : u32x4{0, 0, 0, 0};
+    }
   }
 };
 
@@ -1077,7 +1084,7 @@ __device__ __forceinline__ void pingpong_item(const AttnArgs &a, const int item,
   wait_vmem_all();
   __syncthreads();
   u32x4 qf[8];
-  QTile<L>::read(qf, qtile, L::k_base(l32, g));
+  QTile<L>::read(qf, qtile, L::k_base(l32, g), kSparse || qrow < a.Sq);
   if constexpr (kSparse && !kKeySplit) {
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) pin(qf[ks]);
