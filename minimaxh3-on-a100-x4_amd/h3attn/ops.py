@@ -29,6 +29,9 @@ _SAME_DEVICE = contextlib.nullcontext()
 
 
 def _stream(t: torch.Tensor) -> int:
+    # A CPU tensor's device index is -1, which torch takes for the current GPU.
+    if not t.is_cuda:
+        raise ValueError(f"expected a GPU tensor, got one on {t.device}")
     if _raw_stream is not None:
         return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream

@@ -54,6 +54,25 @@ def test_ops_validate_before_any_gpu_call():
         h3attn.qk_rmsnorm_rope_(q, q, None, torch.ones(128), torch.ones(128), rot_dim=0)
 
 
+def test_cpu_tensors_never_reach_the_library(monkeypatch):
+    """The one-wave fragment tests check only shapes before they ask for the stream, and a stream
+    looked up by device index (-1 for the CPU) would be the current GPU's."""
+    from h3attn import ops
+    monkeypatch.setattr(ops, "_raw_stream", lambda device: 0)
+    monkeypatch.setattr(ops, "check", lambda *a: None)
+
+    class Lib:
+        def __getattr__(self, name):
+            return lambda *a: calls.append(name)
+
+    calls = []
+    monkeypatch.setattr(ops, "lib", Lib)
+    for fn, k in ((ops.test_qk, 128), (ops.test_pv, 64)):
+        with pytest.raises(ValueError, match="GPU"):
+            fn(torch.zeros(32, k), torch.zeros(64, 128))
+    assert not calls
+
+
 def test_rope_table_layout():
     t = h3attn.rope_freqs(10, 64)
     assert tuple(t.shape) == (1, 10, 1, 32, 2, 2) and t.dtype == torch.float32
