@@ -172,12 +172,15 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_kernel(RopeArgs a) {
 // order and combines the four lane groups in that association, so the means
 // are equal to its output bit for bit, and the selection made from them is
 // the same.  Bound by HBM at full size and by the latency of a wave's serial
-// tokens at small ones, so the loads of the next kDepth tokens are in flight
-// while one is computed (they come before its stores, which the compiler cannot
-// reorder) and the cross-lane steps stay in the VALU.  Per call, against loads,
-// LDS shuffles and stores token by token: H=14 S=4104 45.1 -> 24.7 us, H=56 S=4104
-// 67.2 -> 55.8, H=28 S=42120 (blocks of 96) 299 -> 266, H=56 S=42120 510 -> 501
-// (4.9 TB/s; a 2 GiB copy moves 5.0 on the same card).
+// tokens at small ones.  A ring holds kDepth tokens' loads; a slot is refilled
+// after its token's stores (the compiler cannot move loads above them), so
+// with kDepth = 2 one token's loads are in flight while the other is computed, and
+// with 1 none are: there the gain is from cross-lane steps in the VALU and, at
+// rot = 128, a row without branches.  Per call, against LDS shuffles and branches
+// token by token: H=14 S=4104 44.8 -> 24.1 us (4 heads, kDepth = 2), H=56 S=4104
+// 66.9 -> 55.2, H=28 S=42120 (blocks of 96) 299 -> 264, H=56 S=42120 510 -> 499 (4.9
+// TB/s; a 2 GiB copy moves 5.0 on the same card); slower by 2 to 3 % only at rot =
+// 64 with 14 or 28 heads of S=42120.
 template <int kHeadsPerWave, int kDepth, bool kRot128>
 __global__ void __launch_bounds__(256) qk_rmsnorm_rope_pool_kernel(RopeArgs a, int blk, int nb, float *pq,
                                                                    float *pk) {
@@ -209,8 +212,10 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_pool_kernel(RopeArgs a, i
     for (int e = 0; e < 8; ++e) sq[i][e] = sk[i][e] = 0.f;
 
   // This wave's tokens wave, wave + 4, ...: a ring of kDepth tokens' loads in
-  // flight, each slot refilled once its token is done.  Loads past the wave's
-  // last token repeat it (its own rows), so they need no branch.
+  // flight, each slot refilled once its token is done.  With two slots, loads
+  // past the wave's last token repeat it (its own rows): a branch there would
+  // make the compiler wait for both slots (H=14 S=4104: 24.1 us, 30.6 with it).  With
+  // one, the branch costs nothing and the repeated load up to 17 % (blocks of 32).
   const int mine = (rows - wave + 3) / 4;
   struct Token {
     float2 R[8];
@@ -263,7 +268,7 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_pool_kernel(RopeArgs a, i
 #pragma unroll
       for (int d = 0; d < kDepth; ++d) {
         if (n + d < mine) process(ring[d], n + d);
-        load(ring[d], n + d + kDepth);
+        if (kDepth > 1 || n + 1 < mine) load(ring[d], n + d + kDepth);
       }
     }
   }
@@ -309,31 +314,19 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_pool_kernel(RopeArgs a, i
 // Heads per workgroup.  A workgroup's waves walk their share of the block's
 // tokens one after another, so with fewer 8-head workgroups than CUs the launch
 // takes as long as one walk: 4-head chunks double the workgroups and shorten each
-// step.  Measured with 8 / 4 heads: 28.6 / 21.0 us at H=4 S=1024 (16 workgroups of
-// 8 heads), 33.3 / 27.8 at H=14 S=4104 (130), but 55.8 / 79.0 at H=56 S=4104 (455)
-// and 490 / 655 at H=56 S=42120 (4613), where 2 KiB per access of a token's q or k
+// step.  Measured with 8 / 4 heads: 24.5 / 19.5 us at H=4 S=1024 (16 workgroups of
+// 8 heads), 29.3 / 24.1 at H=14 S=4104 (130), but 55.2 / 73.9 at H=56 S=4104 (455)
+// and 499 / 626 at H=56 S=42120 (4613), where 2 KiB per access of a token's q or k
 // against 1 KiB decides.
 constexpr int64_t kPoolWideWgs = 256;
-// With rot = 128 the row needs no branches, and from four workgroups per CU on the
-// 8-head form keeps two tokens in flight (its registers hold fewer workgroups on
-// a CU, which a launch of one or two rounds feels): one token and branches / two
-// tokens without, H=28 S=42120 (1756 workgroups) 269.7 / 265.6 us, H=56 S=24000 in
-// blocks of 128 (1316) 324 / 316, but H=28 S=10000 (420) 72.3 / 75.0 and H=28 S=8192
-// (512) 55.4 / 56.4.  4 heads, with branches / without: 28.1 / 24.7 us at H=14
-// S=4104, 21.0 / 19.4 at H=4 S=1024.
-constexpr int64_t kPoolDeepWgs = 1024;
 int launch_qk_rmsnorm_rope_pool(const RopeArgs &a, int blk, float *pq, float *pk, hipStream_t s) {
   const int nb = (a.S + blk - 1) / blk;
   const int64_t blocks = (int64_t)a.B * nb, wide = blocks * ((a.H + 7) / 8);
-  const bool full = a.rot == kRopeD;
-  auto *kernel = qk_rmsnorm_rope_pool_kernel<8, 1, false>;
-  int64_t wgs = wide;
-  if (wide < kPoolWideWgs) {
-    kernel = full ? qk_rmsnorm_rope_pool_kernel<4, 2, true> : qk_rmsnorm_rope_pool_kernel<4, 2, false>;
-    wgs = blocks * ((a.H + 3) / 4);
-  } else if (full && wide >= kPoolDeepWgs) {
-    kernel = qk_rmsnorm_rope_pool_kernel<8, 2, true>;
-  }
+  const bool full = a.rot == kRopeD, wide_heads = wide >= kPoolWideWgs;
+  auto *kernel = wide_heads
+                     ? (full ? qk_rmsnorm_rope_pool_kernel<8, 1, true> : qk_rmsnorm_rope_pool_kernel<8, 1, false>)
+                     : (full ? qk_rmsnorm_rope_pool_kernel<4, 2, true> : qk_rmsnorm_rope_pool_kernel<4, 2, false>);
+  const int64_t wgs = wide_heads ? wide : blocks * ((a.H + 3) / 4);
   hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(256), 0, s, a, blk, nb, pq, pk);
   return check_launch("qk_rmsnorm_rope_pool_kernel");
 }
