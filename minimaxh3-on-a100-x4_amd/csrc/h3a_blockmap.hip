@@ -350,13 +350,15 @@ __global__ void __launch_bounds__(NW * 64, NW == kSelMidWaves ? 4 : 1) block_sel
 // with one ballot per 64 columns.  Entries past the count are -1.
 //
 // Latency-bound: each 64 columns are a chain of map bytes, ballot and store, and
-// every byte comes from L2.  So four chunks' bytes are loaded at a time, a map
+// every byte comes from L2.  So four chunks' bytes are loaded at a time (while
+// three or four are left; always four took 4.6 us against 3.5 at 4 heads of S=1100 in
+// 16x16 blocks, whose rows are one chunk), a map
 // row that serves several of the sub-block's 16-row slices is read once (a
 // 64-row sub-block spans 1 or 2 map rows from blk_q = 64 on), the second half
 // of a column is read only where it can lie in another key block (blk_k not a
 // multiple of 32), and key blocks are found by a multiplication (block_of_unit).  At H=28,
-// S=42120, 96x96: 47 us, against 98 with eight loads and two divisions per
-// column, one chunk at a time.
+// S=42120, 96x96: 40 us, against 93 with eight loads and two divisions per
+// column, one chunk at a time; 7.2 against 10.2 at S=10000.
 constexpr int kTileUnroll = 4;
 __global__ void __launch_bounds__(256) block_map_to_tile_lut_kernel(const uint8_t *map, int64_t rows, int nsub,
                                                                     int nq, int nk, int Sq, int Skv, int blk_q,
@@ -399,18 +401,20 @@ __global__ void __launch_bounds__(256) block_map_to_tile_lut_kernel(const uint8_
   const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   int32_t *out = lut + row * (int64_t)max_tiles;
   int base = 0;
-  for (int c = 0; c < ncols; c += 64 * kTileUnroll) {
-    uint32_t mask[kTileUnroll];
+  // Columns c .. c + 64 * NU - 1.
+  auto chunks = [&](auto nu_const, int c) __attribute__((always_inline)) {
+    constexpr int NU = decltype(nu_const)::value;
+    uint32_t mask[NU];
 #pragma unroll
-    for (int u = 0; u < kTileUnroll; ++u) mask[u] = 0;
-    // Distinct map rows, wave-uniform: the loads of a row's kTileUnroll chunks are independent.
+    for (int u = 0; u < NU; ++u) mask[u] = 0;
+    // Distinct map rows, wave-uniform: the loads of a row's NU chunks are independent.
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
       if (d >= nd) break;
       const uint8_t *m = mrow[d];
-      uint8_t v0[kTileUnroll], v1[kTileUnroll];
+      uint8_t v0[NU], v1[NU];
 #pragma unroll
-      for (int u = 0; u < kTileUnroll; ++u) {
+      for (int u = 0; u < NU; ++u) {
         const int col = c + 64 * u + lane;
         const int unit = 2 * (col < ncols ? col : 0);  // 16-key units; column 0 is always inside the map
         v0[u] = m[block_of_unit(unit, magic)];
@@ -418,11 +422,11 @@ __global__ void __launch_bounds__(256) block_map_to_tile_lut_kernel(const uint8_
         if (halves) v1[u] = 16 * unit + 16 < Skv ? m[block_of_unit(unit + 1, magic)] : (uint8_t)0;
       }
 #pragma unroll
-      for (int u = 0; u < kTileUnroll; ++u)
+      for (int u = 0; u < NU; ++u)
         mask[u] |= (v0[u] ? bits[d] : 0u) | (v1[u] ? bits[d] << 1 : 0u);
     }
 #pragma unroll
-    for (int u = 0; u < kTileUnroll; ++u) {
+    for (int u = 0; u < NU; ++u) {
       const int col = c + 64 * u + lane;
       uint32_t mk = col < ncols ? mask[u] : 0u;
       if (32 * col + 16 >= Skv) mk &= 0x55u;  // no keys in the column's second half
@@ -431,7 +435,11 @@ __global__ void __launch_bounds__(256) block_map_to_tile_lut_kernel(const uint8_
       if (mk != 0 && pos < max_tiles) out[pos] = (int32_t)(((uint32_t)col << 8) | mk);
       base += __builtin_popcountll(mm);
     }
-  }
+  };
+  int c = 0;
+  for (; c + 128 < ncols; c += 64 * kTileUnroll)  // three chunks and more left
+    chunks(std::integral_constant<int, kTileUnroll>{}, c);
+  for (; c < ncols; c += 64) chunks(std::integral_constant<int, 1>{}, c);
   const int kept = base < max_tiles ? base : max_tiles;
   for (int j = kept + lane; j < max_tiles; j += 64) out[j] = -1;
   if (lane == 0) counts[row] = kept;
