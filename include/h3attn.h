@@ -94,10 +94,10 @@ int h3a_attn_fwd(const void *q, const void *k, const void *v, void *o,
  * queues (1 KiB of counters in the workspace, cleared by the call itself
  * with a kernel before the attention launch), and problems of few tiles may
  * run on shorter ones, whole or split.  h3a_attn_fwd_workspace_size gives the
- * bytes needed for a problem on the current device.  0: workspace may be NULL;
- * that is so for the problems whose 256-row tiles would be neither split nor
- * queued, whichever tiles run.  For the others it is never 0, also where the
- * shorter tiles that run are not split.  The workspace must stay untouched until the call's
+ * bytes to give for a problem on the current device (0: workspace may be
+ * NULL).  Problems whose 256-row tiles would be neither split nor queued never
+ * need one: a NULL or short workspace makes them run unsplit tiles.  The others
+ * always do, also where the shorter tiles that run are not split.  The workspace must stay untouched until the call's
  * work on `stream` has completed, and two calls in flight at once need two
  * workspaces.  Same arguments and errors as h3a_attn_fwd, plus
  * H3A_ERR_INVALID_ARG for a missing or short workspace.  This entry point has

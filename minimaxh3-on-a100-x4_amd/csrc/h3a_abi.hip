@@ -169,7 +169,8 @@ int h3a_attn_fwd_noalloc(const void *q, const void *k, const void *v, void *o, i
   int rc = check_attn(q, k, v, o, B, H, Sq, Skv, D, q_strides, k_strides, v_strides, o_strides, scale);
   if (rc) return rc;
   SplitPlan plan;
-  rc = plan_attn_split(B, H, Sq, Skv, &plan);
+  rc = plan_attn_split(B, H, Sq, Skv, true, &plan);
+  if (!rc && plan.optional && plan.bytes > kScratchBytes) rc = plan_attn_split(B, H, Sq, Skv, false, &plan);
   if (rc) return rc;
   void *ws = nullptr;
   if (plan.bytes > 0) {
@@ -191,7 +192,7 @@ int h3a_attn_fwd_workspace_size(int B, int H, int Sq, int Skv, int D, size_t *by
     return fail(H3A_ERR_INVALID_ARG, "sizes must be positive (B=%d H=%d Sq=%d Skv=%d)", B, H, Sq, Skv);
   if (D != 128) return fail(H3A_ERR_UNSUPPORTED, "head_dim %d unsupported (only 128)", D);
   SplitPlan plan;
-  const int rc = plan_attn_split(B, H, Sq, Skv, &plan);
+  const int rc = plan_attn_split(B, H, Sq, Skv, true, &plan);
   if (rc) return rc;
   *bytes = plan.bytes;
   return H3A_OK;
@@ -205,7 +206,9 @@ int h3a_attn_fwd_ws(const void *q, const void *k, const void *v, void *o, int B,
   int rc = check_attn(q, k, v, o, B, H, Sq, Skv, D, q_strides, k_strides, v_strides, o_strides, scale);
   if (rc) return rc;
   SplitPlan plan;
-  rc = plan_attn_split(B, H, Sq, Skv, &plan);
+  rc = plan_attn_split(B, H, Sq, Skv, true, &plan);
+  if (!rc && plan.optional && (!workspace || workspace_bytes < plan.bytes || !aligned16(workspace)))
+    rc = plan_attn_split(B, H, Sq, Skv, false, &plan);
   if (rc) return rc;
   if (plan.bytes > 0) {
     if (!workspace || workspace_bytes < plan.bytes)

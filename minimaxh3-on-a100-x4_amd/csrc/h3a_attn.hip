@@ -1821,7 +1821,7 @@ static int plan_tiles(int64_t tiles, int stages, bool splittable, bool queued, S
     if (pieces > max_pieces) pieces = max_pieces;
   }
   const int clamped = (int)(tiles > INT_MAX ? INT_MAX : tiles);
-  *plan = SplitPlan{clamped, clamped, 1, 0, false, 0, false, 256};
+  *plan = SplitPlan{clamped, clamped, 1, 0, false, 0, false, 256, false};
   if (tiles > INT_MAX) return H3A_OK;
   if (pieces >= 2) {
     plan->first = (int)(tiles - r);
@@ -1866,27 +1866,29 @@ constexpr int kCombineCycles = 8500, kCombineCyclesPerMB = 600;
 // 59.0, B=32 H=14 Sq=97 Skv=108 16.4 / 18.9 / 25.4, B=32 H=14 S=475 88.8 / 99.1 / 126.2,
 // H=52 Sq=2860 Skv=1003 88.2 / 93.7 / 114.1.
 //
-// Whether a call needs a workspace at all does not depend on the form: a launch
-// whose 256-row tiles would be neither split nor queued needs none, so its
-// shorter forms are not either (one head of S=33000 would run 128-row tiles in
-// ranges otherwise), and one whose 256-row tiles would be asks for
-// kMinWorkspace even where the form that runs writes nothing there.
-int plan_attn_split(int B, int H, int Sq, int Skv, SplitPlan *plan) {
+// Whether a call needs a workspace at all does not depend on the form.  A launch
+// whose 256-row tiles would be neither split nor queued needs none: where a
+// shorter form does better with one (4 heads of 8335 rows and 31366 keys, 128-row
+// tiles in ranges, 466 us against 498) the plan is `optional`, and without
+// `workspace` the best form that uses none is taken.  A launch whose 256-row tiles
+// would be asks for kMinWorkspace even where the form that runs writes nothing
+// there.
+int plan_attn_split(int B, int H, int Sq, int Skv, bool workspace, SplitPlan *plan) {
   int cus = 0;
   int rc = device_cu_count(&cus);
   if (rc) return rc;
   constexpr size_t kMinWorkspace = 256;
   const int stages = (Skv + kBN - 1) / kBN;
   int64_t best = -1;
-  bool bare = false;  // no workspace
+  bool bare = false;  // 256-row tiles use no workspace
   for (const DenseForm &f : kDenseForms) {
     const int64_t tiles = (int64_t)B * H * (((int64_t)Sq + f.rows - 1) / f.rows);
     if (tiles > INT_MAX && f.rows != 256) continue;
     SplitPlan p;
-    rc = plan_tiles(tiles, stages, !bare, true, &p);
+    rc = plan_tiles(tiles, stages, workspace || !bare, true, &p);
     if (rc) return rc;
     if (f.rows == 256) bare = p.bytes == 0;
-    if (bare && p.bytes > 0) continue;
+    if (bare && !workspace && p.bytes > 0) continue;
     // Cycles of a round of items of n stages on `busy` CUs, in cycles of a full
     // chip's clock: the power limit holds 256 busy CUs at about 1.7 GHz, and
     // fewer run faster, up to 2.35 GHz (72 % of the time) at 184 CUs and less.
@@ -1918,6 +1920,7 @@ int plan_attn_split(int B, int H, int Sq, int Skv, SplitPlan *plan) {
     }
   }
   if (!bare && plan->bytes == 0) plan->bytes = kMinWorkspace;
+  plan->optional = bare && plan->bytes > 0;
   return H3A_OK;
 }
 

@@ -81,11 +81,12 @@ struct SplitPlan {
   size_t sched_off;  // byte offset of the queue counters in the workspace
   bool pair_map;     // tile path: sub-blocks paired by stage count (map at offset 0)
   int rows;          // dense: tile height (256, 128 or 64); block-sparse: 64 for one 64-row block per workgroup
+  bool optional;     // dense: a call without the workspace is not refused but planned without one
 };
 
 // Launchers implemented in h3a_attn.hip / h3a_prologue.hip.
 int launch_attn_dense(AttnArgs a, hipStream_t s);  // sets nqt/total from its tile height
-int plan_attn_split(int B, int H, int Sq, int Skv, SplitPlan *plan);
+int plan_attn_split(int B, int H, int Sq, int Skv, bool workspace, SplitPlan *plan);
 int launch_attn_dense_split(AttnArgs a, const SplitPlan &plan, void *ws, hipStream_t s);
 // tiles: a.lut is a tile LUT (column << 8 | sub-block mask per entry) over
 // 64-row query sub-blocks and 32-key columns; blk_q is then ignored.
