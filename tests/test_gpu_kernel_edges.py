@@ -116,11 +116,12 @@ def test_short_tiles_and_key_ranges_match_whole_tiles(gpu, H, Sq, Skv):
     assert d.max() <= 1e-2 * want.abs().max() and d.mean() <= 2.0 ** -7 * want.abs().mean()
 
 
-@pytest.mark.parametrize("H,Sq", [(1, 64), (3, 4000)])
-def test_short_tiles_wide_kv_stride(gpu, H, Sq):
-    """K/V whose rows lie so far apart that a slice passes 2^32 bytes (per-stage descriptors)."""
+@pytest.mark.parametrize("H,Sq,Skv,stride", [(1, 64, 200, (1 << 23) + 8), (3, 4000, 200, (1 << 23) + 8),
+                                             (28, 700, 600, (1 << 22) + 8)])
+def test_short_tiles_wide_kv_stride(gpu, H, Sq, Skv, stride):
+    """K/V whose rows lie so far apart that a slice passes 2^32 bytes (per-stage descriptors), in 64- and
+    (the last) 128-row tiles."""
     torch.manual_seed(1)
-    Skv, stride = 200, (1 << 23) + 8
     buf = torch.empty(Skv * stride, dtype=torch.bfloat16, device=gpu)
     q = torch.randn(1, H, Sq, 128, device=gpu).bfloat16()
     k, v = (torch.randn(1, H, Skv, 128, device=gpu).bfloat16() for _ in range(2))
@@ -128,6 +129,33 @@ def test_short_tiles_wide_kv_stride(gpu, H, Sq):
     kw.copy_(k)
     vw.copy_(v)
     assert torch.equal(ops.attn_fwd(q, kw, vw), ops.attn_fwd(q, k, v))
+
+
+@pytest.mark.parametrize("B,H,Sq,Skv,rows,split", [(32, 48, 26, 73, 64, False), (32, 35, 22, 449, 64, True),
+                                                   (32, 34, 100, 198, 128, False), (32, 35, 74, 576, 128, True)])
+def test_short_tiles_queued(gpu, B, H, Sq, Skv, rows, split):
+    """Four rounds and more of 128- and 64-row tiles on the persistent grid, where an item's query rows land
+    in the buffers of the last one's exchange, alone and followed by a split tail: equal to the unsplit
+    256-row tiles within rounding, to the oracle on the last head, and to itself over garbage counters."""
+    if torch.cuda.get_device_properties(gpu).multi_processor_count != 256:
+        pytest.skip("the shapes are chosen for 256 CUs")
+    tiles = B * H * -(-Sq // rows)
+    need = ops.attn_workspace_bytes(B, H, Sq, Skv)
+    one = tiles % 256 * rows * 130 * 4  # partials of one range of each tail tile
+    assert tiles >= 1024 and (need - 1024 >= 2 * one and (need - 1024) % one == 0 if split else need == 1024)
+    rng = np.random.default_rng(Sq + Skv)
+    q, k, v = (randn_bf16(rng, (B, H, n, 128)) for n in (Sq, Skv, Skv))
+    dev = [to_dev_bf16(x, gpu) for x in (q, k, v)]
+    outs = []
+    for fill in (0, 0x7F):
+        torch.full((need,), fill, dtype=torch.uint8, device=gpu)  # freed: the next workspace's bytes
+        outs.append(ops.attn_fwd(*dev))
+    assert torch.equal(*outs)
+    want = ops.attn_fwd(*dev, split_tail=False).float()
+    d = (outs[0].float() - want).abs()
+    assert d.max() <= 1e-2 * want.abs().max() and d.mean() <= 2.0 ** -7 * want.abs().mean()
+    got = oracle.bf16_to_f32(from_dev_bf16(outs[0][-1:, -1:].contiguous())).reshape(1, 1, Sq, 128)
+    assert_close_absmax(got, oracle.attn_fwd(*(x[-1:, -1:] for x in (q, k, v))), what=f"{rows}-row tiles, queued")
 
 
 @pytest.mark.parametrize("H,nq,nk", [(1, 1, 1), (2, 5, 64), (3, 17, 128), (14, 65, 65), (4, 33, 129), (60, 65, 65),
@@ -152,10 +180,12 @@ def test_block_select_rows_per_workgroup(gpu, H, nq, nk):
 
 @pytest.mark.parametrize("H,blk_q,blk_k,Sq,Skv", [(1, 64, 64, 64, 64), (2, 64, 64, 333, 1000), (3, 64, 128, 1000, 1090),
                                                   (2, 64, 256, 640, 2500), (2, 192, 64, 700, 1100),
-                                                  (4, 192, 192, 4096, 777), (5, 64, 64, 4096, 333)])
+                                                  (4, 192, 192, 4096, 777), (5, 64, 64, 4096, 333),
+                                                  (4, 64, 64, 4096, 1300), (5, 64, 64, 4096, 1300)])
 def test_one_sparse_block_per_workgroup(gpu, H, blk_q, blk_k, Sq, Skv):
-    """64-row query blocks, few enough for one per CU (and, last, just too many): both groups on one block's
-    list, with empty, one-entry and full lists, against the masked oracle."""
+    """64-row query blocks with lists of 8 stages and more, few enough for one per CU (up to the last but
+    one, 256; the last is just too many), and with shorter lists: both groups on one block's list, with
+    empty, one-entry and full lists, against the masked oracle."""
     rng = np.random.default_rng(Sq + Skv)
     q, k, v = (randn_bf16(rng, (1, H, n, 128)) for n in (Sq, Skv, Skv))
     bmap = (rng.random((1, H, -(-Sq // blk_q), -(-Skv // blk_k))) < 0.4).astype(np.uint8)
@@ -169,3 +199,18 @@ def test_one_sparse_block_per_workgroup(gpu, H, blk_q, blk_k, Sq, Skv):
     got = oracle.bf16_to_f32(from_dev_bf16(out)).reshape(out.shape)
     assert_close_absmax(got, oracle.attn_fwd(q, k, v, block_map=bmap, blk_q=blk_q, blk_k=blk_k),
                         what=f"{H} heads {blk_q}x{blk_k}")
+
+
+def test_one_sparse_block_per_workgroup_wide_kv_stride(gpu):
+    """The same with K/V whose rows lie so far apart that a slice passes 2^32 bytes (per-stage descriptors)."""
+    torch.manual_seed(2)
+    Sq, Skv, stride = 200, 600, (1 << 22) + 8  # lists of up to 10 stages
+    buf = torch.empty(Skv * stride, dtype=torch.bfloat16, device=gpu)
+    q = torch.randn(1, 1, Sq, 128, device=gpu).bfloat16()
+    k, v = (torch.randn(1, 1, Skv, 128, device=gpu).bfloat16() for _ in range(2))
+    kw, vw = (buf.as_strided((1, 1, Skv, 128), (0, 128, stride, 1), off * 128) for off in (0, 1))
+    kw.copy_(k)
+    vw.copy_(v)
+    lut, cnt = h3attn.block_map_to_lut((torch.rand(1, 1, 4, 10, device=gpu) < 0.8).to(torch.uint8), 10)
+    assert torch.equal(ops.attn_fwd_blocksparse(q, kw, vw, lut, cnt, 64, 64),
+                       ops.attn_fwd_blocksparse(q, k, v, lut, cnt, 64, 64))
