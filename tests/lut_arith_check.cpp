@@ -65,6 +65,23 @@ int main() {
         }
       }
     }
+  // Key blocks of the tile LUT's 16-key units: every unit it can name, at block
+  // sizes up to and past the largest that the multiplication serves.
+  std::vector<int64_t> bs;
+  for (int b = 1; b <= 300; ++b) bs.push_back(b);
+  for (int64_t b : {65535ll, 65536ll, 65537ll, 131071ll, 131072ll, 174763ll, 262139ll, 262143ll, 262144ll, 262145ll,
+                    1000003ll, (long long)(INT_MAX / 16)})
+    bs.push_back(b);
+  for (int i = 0; i < 100; ++i) bs.push_back(1 + (int64_t)(rng() % (1u << 18)));
+  for (int64_t b : bs) {
+    const uint64_t magic = h3a::unit_magic((int)(16 * b));
+    for (int u = 0; u < 1 << 18; ++u)
+      if (h3a::block_of_unit(u, magic) != u / b) {
+        printf("block_of_unit(%d) = %d at %lld-key blocks, want %lld\n", u, h3a::block_of_unit(u, magic),
+               (long long)(16 * b), (long long)(u / b));
+        return 1;
+      }
+  }
   printf("OK\n");
   return 0;
 }

@@ -2,7 +2,8 @@
 checked against int64 math: the key block of a stage (t / sub, with sub = 3 as a
 multiply-high) and a stage's first key, including LUT entries far outside the key
 range (2^24 + 5, 2^31 - 1, negative), which must map to Skv (load nothing) instead
-of wrapping a 32-bit multiply.  No GPU needed."""
+of wrapping a 32-bit multiply; and the key block of every 16-key unit a tile LUT can
+name.  No GPU needed."""
 from __future__ import annotations
 
 import os
