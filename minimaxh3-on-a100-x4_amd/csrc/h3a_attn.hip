@@ -1781,11 +1781,12 @@ int launch_attn_dense(AttnArgs a, hipStream_t s) {
   return check_launch("attn_fwd_pingpong_kernel<dense>");
 }
 
-// Split-tail plan.  With one workgroup per CU, N whole 256-row tiles run in
+// Split-tail plan.  With one workgroup per CU, N whole tiles run in
 // ceil(N / CUs) rounds and the last round keeps only N % CUs CUs busy (all of
 // the chip idles but N for N < CUs).  Those r tiles are cut into P key
-// ranges each, P = CUs / r (at least kMinSplitStages 64-key stages per
-// range), so the last round is ~1/P as long.
+// ranges each (at least kMinSplitStages 64-key stages per range), so the last
+// round is ~1/P as long: P = CUs / r for block-sparse pairs, up to that for dense
+// tiles (plan_attn_split).
 static int device_cu_count(int *cus_out) {
   static std::atomic<int> cu_cache[64];
   int dev = 0;
@@ -1800,12 +1801,12 @@ static int device_cu_count(int *cus_out) {
   return H3A_OK;
 }
 
-// `tiles` 256-row work items of up to `stages` stages each, split when
+// `tiles` work items of `rows` rows and up to `stages` stages each, split when
 // `splittable`.  With `queued`, problems of at least kQueuedRounds rounds of
 // tiles run on a persistent grid fed by the per-XCD queues (take_item): the
 // XCDs' clocks differ under full load by up to ~5 %, and with a static
 // deal the fastest XCD idles while the slowest finishes its share.
-// `max_pieces` bounds the ranges per tile; `rows` is the tile height.
+// `max_pieces` bounds the ranges per tile.
 static int plan_tiles(int64_t tiles, int stages, bool splittable, bool queued, SplitPlan *plan,
                       int max_pieces = INT_MAX, int rows = 256) {
   constexpr int kMinSplitStages = 4;
@@ -1947,13 +1948,13 @@ int plan_attn_sparse_split(int B, int H, int Sq, int blk_q, int blk_k, int max_k
 
 // The same for a tile LUT (64-row sub-blocks, unsplit): max_tiles entries
 // stand in for the stage count.  The workspace starts with the pair map
-// (tile_pair_map_kernel; up to kPairSortMax sub-blocks per (b,h), beyond
+// (tile_pair_map_kernel; up to kPairMapMax sub-blocks per (b,h), beyond
 // that pairs 2p, 2p+1), then the queue counters.
 int plan_attn_sparse_tiles(int B, int H, int Sq, int max_tiles, SplitPlan *plan) {
   const int64_t nsub = (Sq + 63) / 64;
   const int64_t pairs = (int64_t)B * H * ((nsub + 1) / 2);
   const int rc = plan_tiles(pairs, max_tiles, false, true, plan);
-  if (rc || nsub > kPairSortMax || pairs > INT_MAX) return rc;
+  if (rc || nsub > kPairMapMax || pairs > INT_MAX) return rc;
   const size_t map_bytes = (size_t)pairs * 2 * sizeof(int32_t);
   plan->pair_map = true;
   if (plan->dynamic) {

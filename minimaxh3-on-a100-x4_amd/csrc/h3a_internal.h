@@ -67,8 +67,10 @@ inline bool tile_block_ok(int blk) { return blk > 0 && blk % 16 == 0; }
 // and below 2^24): Skv <= kMaxTileColumns * 32.
 constexpr int kMaxTileColumns = 65534;
 // Query sub-blocks per (b,h) up to which they are paired by stage count (tile
-// path; longer sequences pair sub-blocks 2p, 2p+1).
-constexpr int kPairSortMax = 16384;
+// path; longer sequences pair sub-blocks 2p, 2p+1).  The ranking has no limit of
+// its own: this one is the entry point's, whose workspace for longer sequences is
+// the queues' 1 KiB alone.
+constexpr int kPairMapMax = 16384;
 inline int sparse_sub_block_rows(int blk_q) { return blk_q % 128 == 0 ? 128 : 64; }
 
 // Dense split-tail plan for a problem on the current device.

@@ -698,7 +698,7 @@ def test_sparse_tiles_pair_map(gpu, B, H, S, blk):
 def test_sparse_tiles_pair_map_limit(gpu, extra):
     """Up to 16384 sub-blocks per (b,h) the workspace holds the pair map (8 bytes a pair) and
     the queue counters; one more and the pairs stay consecutive (counters only).  At the
-    limit (S = 64 * 16384, the sort over 16384 sub-blocks of random lengths) and just past
+    limit (S = 64 * 16384, 16384 sub-blocks of random lengths ranked in runs) and just past
     it (S = 64 * 16384 + 1), the queued call equals the plain one bit for bit and fp32
     attention on rows of the first, a middle and the last sub-block.  Sub-block s lists
     its own diagonal column 2s with rows 0-31 admitted, and 0-3 more columns 2s+1 .. with
