@@ -204,12 +204,15 @@ class Schedule:
         return sla.sparse_attention(q, k, v, keep, self.blk, force_diag=self.force_diag, smooth_k=self.smooth_k,
                                     pooled=pooled, seq_major=seq_major)
 
-    def run(self, layer, q, k, v, transformer_options=None, pooled=None, seq_major=False):
+    def run(self, layer, q, k, v, transformer_options=None, pooled=None, seq_major=None):
         """[1,H,S,D] sparse output, or None (keep >= 1: caller runs dense).
 
         pooled: the layer's block means from the prologue, if it took them.
-        seq_major: the output's memory layout (sla.sparse_attention).
+        seq_major: the output's memory layout (sla.sparse_attention); None: sequence-major
+        inside make_sla_override's override, head-major elsewhere.
         """
+        if seq_major is None:
+            seq_major = getattr(_state, "seq_major", False)
         if layer == 0:
             self.generation_start(transformer_options)
         keep = self.keep_for(layer)
@@ -253,8 +256,12 @@ def make_sla_override(topk: float = 0.35, blk: int = 64, schedule: Schedule | No
         pooled = _take_pooled(q, k, blk)
         if schedule is None:
             return sla.sparse_attention(q, k, v, topk, blk, pooled=pooled, seq_major=True)
-        return schedule.run(getattr(_state, "layer", None), q, k, v, transformer_options, pooled=pooled,
-                            seq_major=True)
+        # The layout goes through the thread's state: a caller's own schedule need not know of it.
+        _state.seq_major = True
+        try:
+            return schedule.run(getattr(_state, "layer", None), q, k, v, transformer_options, pooled=pooled)
+        finally:
+            _state.seq_major = False
 
     def plan(layer):
         """(keep, blk) this override applies to DiT layer `layer`."""

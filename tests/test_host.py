@@ -265,6 +265,27 @@ def test_sla_override_scope_schedule_and_fallback():
     assert sched.keep_for(None) == sched.default_keep and sched.keep_for(99) == sched.default_keep
 
 
+def test_sla_override_runs_a_schedule_with_its_own_run(monkeypatch):
+    """A schedule whose run takes only the layer, q, k, v, the options and the pooled means runs sparse
+    under the override (no fallback), and Schedule.run's output is sequence-major there alone."""
+    layouts, logs = [], []
+    monkeypatch.setattr(sla, "sparse_attention",
+                        lambda q, *a, seq_major=False, **kw: layouts.append(seq_major) or q)
+
+    class Own(hooks.Schedule):
+        def run(self, layer, q, k, v, transformer_options=None, pooled=None):
+            return super().run(layer, q, k, v, transformer_options, pooled=pooled)
+
+    sched = Own("custom", [0.5] * 50, blk=64)
+    ov = hooks.make_sla_override(schedule=sched, log=logs.append)
+    q = torch.randn(1, 2, 12, 128)
+    monkeypatch.setattr(hooks, "in_dit_scope", lambda: True)
+    out = ov(lambda *a, **kw: pytest.fail("fell back"), q, q, q, 2, mask=None, skip_reshape=True)
+    assert torch.equal(out, q.transpose(1, 2).reshape(1, 12, 256)) and logs == []
+    sched.run(3, q, q, q)
+    assert layouts == [True, False]
+
+
 def test_sla_block_size_checked_at_construction():
     """Every size the node offers (16..256 step 16, custom_nodes/h3_sla/__init__.py:315) is accepted;
     others fail when the schedule/override is built (as the node fails at patch time, h3_sla:331),
