@@ -29,11 +29,11 @@ _SAME_DEVICE = contextlib.nullcontext()
 
 
 def _stream(t: torch.Tensor) -> int:
-    # A CPU tensor's device index is -1, which torch takes for the current GPU.
-    if not t.is_cuda:
+    device = t.get_device()
+    if device < 0:  # not on a GPU; the lookup would take -1 for the current one
         raise ValueError(f"expected a GPU tensor, got one on {t.device}")
     if _raw_stream is not None:
-        return _raw_stream(t.get_device())
+        return _raw_stream(device)
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
