@@ -179,8 +179,8 @@ __global__ void __launch_bounds__(256) qk_rmsnorm_rope_kernel(RopeArgs a) {
 // rot = 128, a row without branches.  Per call, against LDS shuffles and branches
 // token by token: H=14 S=4104 44.8 -> 24.1 us (4 heads, kDepth = 2), H=56 S=4104
 // 66.9 -> 55.2, H=28 S=42120 (blocks of 96) 299 -> 264, H=56 S=42120 510 -> 499 (4.9
-// TB/s; a 2 GiB copy moves 5.0 on the same card); slower by 2 to 3 % only at rot =
-// 64 with 14 or 28 heads of S=42120.
+// TB/s; a 2 GiB copy moves 5.0 on the same card); longer by more than 1 % (to 3 %)
+// only at rot = 64 with 14 or 28 heads of S=42120.
 template <int kHeadsPerWave, int kDepth, bool kRot128>
 __global__ void __launch_bounds__(256) qk_rmsnorm_rope_pool_kernel(RopeArgs a, int blk, int nb, float *pq,
                                                                    float *pk) {
